@@ -3,8 +3,9 @@
 //   1. preprocess: per query row, lse2 = lse * log2(e) and
 //      ndelta = -rowsum(dout * out) (the `D` term of dS = P * (dP - D)), in
 //      arrays padded to whole 64-row tiles (+inf / 0 past the end so padded
-//      rows get P = 0); plus the padded operand copies (prep.hip): row-major
-//      q and dout, head_dim-major k (and row-major k, v for 3'');
+//      rows get P = 0); plus the padded operand copies (prep.hip):
+//      head_dim-major k (row-major k, v for 3''), and row-major q where it is
+//      rotated first;
 //   2. dK/dV: one workgroup per 128 keys (32 per wave, kept in registers as
 //      MFMA operands); loops over 64-row query tiles of every query head
 //      that reads this KV head; with staged dS it also stores dS (bf16) to
@@ -161,8 +162,13 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
   const int group = a.Hq / a.Hkv;
 
   const int key = kt * BK + kw * 32 + l32;
-  bool kvalid = key < a.Lk;
-  if (MASK && kvalid) kvalid = a.mask[b * a.msb + key] != 0;
+  // Whether this lane's key is attended; read again for the epilogue rather
+  // than held through the loop, which has no register to spare.
+  auto key_valid = [&]() {
+    bool ok = key < a.Lk;
+    if (MASK && ok) ok = a.mask[b * a.msb + key] != 0;
+    return ok;
+  };
 
   // This wave's B operand: K (P waves, rotated when the backward carries the
   // key's rotation) or V (dS waves) of the lane's key, read once from the
@@ -299,11 +305,14 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
   const int niter = ntq * group;
   auto tile_head = [&](int it) { return it / ntq; };     // query head within the group
   auto tile_idx = [&](int it) { return tq0 + it % ntq; };  // 64-row tile of that head
-  // Buffers over the query heads of this KV head's group (b, hk*group ..).
+  // The tiles this wave loads (dO for a P wave, Q for a dS wave), read where
+  // BwdArgs::dt / qt point: the caller's tensor (rows past the end read as
+  // zeros, see tile_rsrc) or a padded copy.
   const int64_t bq0 = (int64_t)(b * a.Hq + hk * group);
-  const uint32_t qbytes = (uint32_t)group * a.Lqp * D * 2;
-  const u32x4 rq = make_rsrc(a.qr + bq0 * a.Lqp * D, qbytes);
-  const u32x4 rdo = make_rsrc(a.dor + bq0 * a.Lqp * D, qbytes);
+  const int64_t th = role == 0 ? a.dth : a.qth;
+  const int tl = (int)(role == 0 ? a.dtl : a.qtl);
+  const bf16* t00 = role == 0 ? a.dt + b * a.dtb : a.qt + b * a.qtb;
+  t00 += (int64_t)hk * group * th;
   const u32x4 rl2 = make_rsrc(a.lse2 + bq0 * a.Lqp, (uint32_t)group * a.Lqp * 4);
   const u32x4 rnd = make_rsrc(a.ndelta + bq0 * a.Lqp, (uint32_t)group * a.Lqp * 4);
   // A tile is loaded in two parts, one load at a time between MFMAs (a burst
@@ -311,12 +320,20 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
   // stream): the dS waves load its Q rows (kQOps loads per wave) during their
   // dP phase of the iteration before, the P waves its dO rows and statistics
   // (kROps) during their dV phase of the iteration before that.
-  TileStager<BQ, D, 4> rst;  // 64 rows of D channels (row stride D) over 4 waves
-  rst.init(D, kw, lane);
+  TileStager<BQ, D, 4> rst;  // 64 rows of D channels (row stride tl) over 4 waves
+  rst.init(tl, kw, lane);
   constexpr int kQOps = TileStager<BQ, D, 4>::kPer;
   constexpr int kROps = kQOps + 2 + (WIN ? 2 : 0);
-  auto tile_rows = [&](int it) {  // first row of tile `it` in the group's copies
+  auto tile_rows = [&](int it) {  // first row of tile `it` in the group's statistics
     return (uint32_t)tile_head(it) * a.Lqp + (uint32_t)tile_idx(it) * BQ;
+  };
+  // Buffer over tile `it`'s rows of this wave's source: from its first row to
+  // the end of its last valid one, so that loads of rows past the end (tl >=
+  // D, so they start past the range) return zeros.
+  auto tile_rsrc = [&](int it) {
+    const int row0 = tile_idx(it) * BQ;
+    const int last = min(a.Lq - 1 - row0, BQ - 1);
+    return make_rsrc(t00 + tile_head(it) * th + (int64_t)row0 * tl, (uint32_t)(last * tl + D) * 2);
   };
   // Window arrays of this batch (WIN); rows past Lq read as 0 (empty).
   u32x4 rwl = {0u, 0u, 0u, 0u}, rwh = {0u, 0u, 0u, 0u};
@@ -324,17 +341,16 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
     rwl = make_rsrc(a.wlo + b * a.wsb, (uint32_t)a.Lq * 4);
     rwh = make_rsrc(a.whi + b * a.wsb, (uint32_t)a.Lq * 4);
   }
-  // Q load i of tile `it` into Q slot `qd`.
-  auto q_op = [&](int it, bf16* qd, int i) { rst.stage_one(qd, rq, tile_rows(it) * D * 2, i); };
-  // Row load i of tile `it` into row slot `rsg`.
-  auto r_op = [&](int it, RowStage& rsg, int i) {
-    const uint32_t row0 = tile_rows(it);
+  // Q load i of a tile (its buffer rq) into Q slot `qd`.
+  auto q_op = [&](const u32x4& rq, bf16* qd, int i) { rst.stage_one(qd, rq, 0u, i); };
+  // Row load i of tile `it` (its dO buffer rdo) into row slot `rsg`.
+  auto r_op = [&](int it, const u32x4& rdo, RowStage& rsg, int i) {
     if (i < kQOps)
-      rst.stage_one(rsg.dout, rdo, row0 * D * 2, i);
+      rst.stage_one(rsg.dout, rdo, 0u, i);
     else if (i == kQOps)
-      dma4(rl2, lds_addr(rsg.lse2), lane * 4, row0 * 4);  // every wave loads the stats: no branch
+      dma4(rl2, lds_addr(rsg.lse2), lane * 4, tile_rows(it) * 4);  // every wave loads the stats: no branch
     else if (i == kQOps + 1)
-      dma4(rnd, lds_addr(rsg.ndl), lane * 4, row0 * 4);
+      dma4(rnd, lds_addr(rsg.ndl), lane * 4, tile_rows(it) * 4);
     else if (i == kQOps + 2)
       dma4(rwl, lds_addr(rsg.wlo), lane * 4, (uint32_t)tile_idx(it) * BQ * 4);
     else
@@ -361,7 +377,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
   // of dS as four 16-byte stores per lane (group g = 2*sub + k2: the lane's
   // key, its 8 consecutive rows), each instruction 1 KB contiguous in unit
   // `sub`, in the first slot of each group's dK^T MFMAs.
-  const uint32_t ds_keep = kvalid ? 0xffffffffu : 0u;  // dS of masked / past-the-end keys is stored as 0
+  const uint32_t ds_keep = STAGE && key_valid() ? 0xffffffffu : 0u;  // dS of masked / past-the-end keys is stored as 0
   const uint32_t ds_voff = DsUnit::store_offset(kw * 32 + l32, lane, 0, 0, 0);
 
   const float c = a.scale_log2;
@@ -484,6 +500,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
     bf16x8 opq[kRA];
 #pragma unroll
     for (int j = 0; j < kRA; ++j) opq[j] = dot_op(j);
+    const u32x4 lrd = tile_rsrc(itr);  // scalar work, here behind the first reads' latency
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
@@ -491,11 +508,11 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
       if (j + kRA < NJ) opq[j % kRA] = dot_op(j + kRA);
       const int sk = j / DT, dt = j % DT;
       acc[dt] = mfma32(op, pb[sk >> 1][sk & 1], acc[dt]);
-      if (load_slot(j, NJ, kROps)) r_op(itr, lrs, j - kLoad0);
+      if (load_slot(j, NJ, kROps)) r_op(itr, lrd, lrs, j - kLoad0);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int i = loads_in_loop(NJ); i < kROps; ++i) r_op(itr, lrs, i);
+    for (int i = loads_in_loop(NJ); i < kROps; ++i) r_op(itr, lrd, lrs, i);
   };
 
   // dS waves, dP phase of the tile in slot uc: dp = dO V^T + ndelta, and the
@@ -518,6 +535,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
     };
 #pragma unroll
     for (int q4 = 0; q4 < 4; ++q4) nd_read(0, q4);
+    const u32x4 lrq = tile_rsrc(itq);  // scalar work, here behind the first reads' latency
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
@@ -525,11 +543,11 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
       dp[sub] = mfma32(da[j % kRA], kv[ks], dp[sub]);
       if (j + kRA < NS) da[j % kRA] = dop(j + kRA);
       if (j < 4) nd_read(1, j);  // KS >= 4: before sub 1's first MFMA
-      if (load_slot(j, NS, kQOps)) q_op(itq, lq, j - kLoad0);
+      if (load_slot(j, NS, kQOps)) q_op(lrq, lq, j - kLoad0);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int i = loads_in_loop(NS); i < kQOps; ++i) q_op(itq, lq, i);
+    for (int i = loads_in_loop(NS); i < kQOps; ++i) q_op(lrq, lq, i);
   };
 
   // Where tile `it`'s dS goes (STAGE): a buffer over its two units (query
@@ -645,12 +663,12 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
   retire_prologue_loads();
   if (niter > 0 && role == 0) {  // niter is 0 when no window meets this block's keys
 #pragma unroll
-    for (int i = 0; i < kROps; ++i) r_op(0, sm.rs[0], i);
+    for (int i = 0; i < kROps; ++i) r_op(0, tile_rsrc(0), sm.rs[0], i);
 #pragma unroll
-    for (int i = 0; i < kROps; ++i) r_op(min(1, niter - 1), sm.rs[1], i);
+    for (int i = 0; i < kROps; ++i) r_op(min(1, niter - 1), tile_rsrc(min(1, niter - 1)), sm.rs[1], i);
   } else if (niter > 0) {
 #pragma unroll
-    for (int i = 0; i < kQOps; ++i) q_op(0, sm.q[0], i);
+    for (int i = 0; i < kQOps; ++i) q_op(tile_rsrc(0), sm.q[0], i);
   }
   // Tile it lives in slot it % 3 (Q, rows and P hand-over); the loops are
   // unrolled by 3 so that every slot is a compile-time constant.  Every wave
@@ -701,6 +719,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
     }
   }
 
+  const bool kvalid = key_valid();
   if (part >= 0) {
     // Unscaled fp32 partial sums (masked keys and keys past the end as 0);
     // dkv_reduce_kernel scales, rounds and rotates their total.
@@ -1353,20 +1372,41 @@ static void launch_dq_ds_d(const BwdArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL((bwd_dq_ds_kernel<D, 64, 3, false, false>), grid, dim3(512), 0, stream, a);
 }
 
+// Whether the dK/dV kernel can read 64-row tiles of rows `row_stride` elements
+// apart in place: rows that do not overlap (so that a row past the end starts
+// past the tile's buffer range) and a tile span within 32-bit byte offsets.
+static bool tiles_in_place(int64_t row_stride, int D) { return row_stride >= D && row_stride < (int64_t)1 << 23; }
+
 template <int D>
-static hipError_t launch_bwd_d(const BwdArgs& a, int kv_per_pass, hipStream_t stream) {
+static hipError_t launch_bwd_d(const BwdArgs& args, int kv_per_pass, hipStream_t stream) {
+  BwdArgs a = args;
   const bool mask = a.mask != nullptr;
+  // Sources of the dK/dV kernel's Q and dO tiles: the caller's tensors, or
+  // padded copies where q is rotated first or the rows cannot be read in
+  // place.  A copy is one read and one write of the tensor at HBM rate, which
+  // the tile loads then repeat: without the two of them 75,600 queries x 512
+  // keys (2 x 40 heads, D 128) went from 8.53 to 7.35 ms forward + backward,
+  // a 13x15x27-token block from 1.218 to 1.192 ms; at 16k tokens the copies
+  // are under 1% of the step.
+  const int64_t ch = (int64_t)a.Lqp * D;  // a copy's head stride
+  if (a.cos_q == nullptr && tiles_in_place(a.qsl, D)) {
+    a.qt = a.q, a.qtb = a.qsb, a.qth = a.qsh, a.qtl = a.qsl;
+  } else {
+    a.qt = a.qr, a.qtb = a.Hq * ch, a.qth = ch, a.qtl = D;
+  }
+  if (tiles_in_place(a.dosl, D)) {
+    a.dt = a.dout, a.dtb = a.dosb, a.dth = a.dosh, a.dtl = a.dosl;
+  } else {
+    a.dt = a.dor, a.dtb = a.Hq * ch, a.dth = ch, a.dtl = D;
+  }
   {
     LaunchTimer timer(kKidTranspose, stream);
     hipError_t e = hipSuccess;
-    if (!a.reuse_q) {
-      // Row-major copies only: the dK/dV kernel reads its head_dim-major
-      // operands from the same tiles by transposed LDS reads.
+    if (!a.reuse_q && a.qt == a.qr)
       e = launch_prep_copies(a.q, a.qsb, a.qsh, a.qsl, a.B, a.Hq, a.Lq, D, a.qr, nullptr, stream, nullptr, a.cos_q,
                              a.sin_q, a.rqsb);
-      if (e == hipSuccess)
-        e = launch_prep_copies(a.dout, a.dosb, a.dosh, a.dosl, a.B, a.Hq, a.Lq, D, a.dor, nullptr, stream);
-    }
+    if (e == hipSuccess && !a.reuse_q && a.dt == a.dor)
+      e = launch_prep_copies(a.dout, a.dosb, a.dosh, a.dosl, a.B, a.Hq, a.Lq, D, a.dor, nullptr, stream);
     // The dK/dV kernel reads its own key rows from k and v; the row-major
     // copies serve only the recomputing dQ kernel (no staged dS), the
     // head_dim-major k copy both dQ kernels.

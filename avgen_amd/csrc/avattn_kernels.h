@@ -104,6 +104,13 @@ struct BwdArgs {
   bf16* kr;
   bf16* vr;
   bf16* kt;
+  // Where the dK/dV kernel reads its Q and dO tiles (set by launch_bwd): q and
+  // dout themselves or the copies qr and dor; row i of (b, hq) at b*qtb +
+  // hq*qth + i*qtl (dtb, dth, dtl for dO).
+  const bf16* qt;
+  int64_t qtb, qth, qtl;
+  const bf16* dt;
+  int64_t dtb, dth, dtl;
   float* kbias;  // (B, Lkp): 0 attended / -inf
   int* kfull;    // (B, Lkp/32): 1 if every key of the 32-key tile is attended
   int Lqp, Lkp;
