@@ -31,44 +31,6 @@
 namespace avattn {
 
 // ---------------------------------------------------------------------------
-// 1. lse2 / ndelta
-// ---------------------------------------------------------------------------
-template <int D>
-__global__ __launch_bounds__(256) void bwd_pre_kernel(BwdArgs a) {
-  constexpr int TPR = D / 8;  // threads per row
-  constexpr int RPB = 256 / TPR;
-  const int64_t rows = (int64_t)a.B * a.Hq * a.Lqp;
-  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / TPR;
-  const int c = threadIdx.x % TPR;
-  const int i = (int)(row % a.Lqp);
-  const int64_t bh = row / a.Lqp;
-  const bool valid = row < rows && i < a.Lq;
-  float acc = 0.f;
-  if (valid) {
-    const int h = (int)(bh % a.Hq);
-    const int b = (int)(bh / a.Hq);
-    const u32x4 x = *reinterpret_cast<const u32x4*>(a.dout + b * a.dosb + h * a.dosh + (int64_t)i * a.dosl + 8 * c);
-    const u32x4 y = *reinterpret_cast<const u32x4*>(a.out + b * a.osb + h * a.osh + (int64_t)i * a.osl + 8 * c);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      acc = fmaf(__uint_as_float(x[w] << 16), __uint_as_float(y[w] << 16), acc);
-      acc = fmaf(__uint_as_float(x[w] & 0xffff0000u), __uint_as_float(y[w] & 0xffff0000u), acc);
-    }
-  }
-#pragma unroll
-  for (int off = TPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, TPR);
-  if (row < rows && c == 0) {
-    a.ndelta[row] = -acc;
-    if (valid) {
-      const float l = a.lse[bh * a.Lq + i];
-      a.lse2[row] = (l == kNegInf) ? kPosInf : l * kLog2e;
-    } else {
-      a.lse2[row] = kPosInf;
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // 2. dK / dV
 // ---------------------------------------------------------------------------
 // One workgroup = 128 keys and 8 waves in two roles; waves w and w+4 own the
@@ -296,6 +258,11 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
     }
     w_ia = __builtin_amdgcn_readfirstlane(c_a);
     w_ib = __builtin_amdgcn_readfirstlane(c_b);
+  }
+  // A block outside the pair's hull of contributing tiles (every key masked):
+  // dK and dV are zeros and dS is not read.
+  if (MASK && STAGE && !WIN) {
+    if (2 * kt >= load_const_i32(a.khull, 2 * bhk + 1) || 2 * kt + 2 <= load_const_i32(a.khull, 2 * bhk)) ntq = 0;
   }
   if (part >= 0) {  // this part's share of the tiles (possibly none)
     const int p0 = ntq * part / a.nparts, p1 = ntq * (part + 1) / a.nparts;
@@ -1198,6 +1165,10 @@ __global__ __launch_bounds__(512, 1) void bwd_dq_ds_kernel(BwdArgs a) {
   const int nkt = (a.Lk + 127) / 128;
   int s0 = 0, s1 = a.Lkp / BK;  // stages of the workgroup
   int w0 = s0, w1 = s1;         // stages this wave multiplies
+  if constexpr (!WIN) {
+    s0 = load_const_i32(a.khull, 2 * (b * a.Hkv + hk)) * (64 / BK);
+    s1 = load_const_i32(a.khull, 2 * (b * a.Hkv + hk) + 1) * (64 / BK);
+  }
   if constexpr (WIN) {
     // Monotone windows: a row range's key union is [lo(first), hi(last)).
     const int* lo = a.wlo + b * a.wsb;
@@ -1399,32 +1370,8 @@ static hipError_t launch_bwd_d(const BwdArgs& args, int kv_per_pass, hipStream_t
   } else {
     a.dt = a.dor, a.dtb = a.Hq * ch, a.dth = ch, a.dtl = D;
   }
-  {
-    LaunchTimer timer(kKidTranspose, stream);
-    hipError_t e = hipSuccess;
-    if (!a.reuse_q && a.qt == a.qr)
-      e = launch_prep_copies(a.q, a.qsb, a.qsh, a.qsl, a.B, a.Hq, a.Lq, D, a.qr, nullptr, stream, nullptr, a.cos_q,
-                             a.sin_q, a.rqsb);
-    if (e == hipSuccess && !a.reuse_q && a.dt == a.dor)
-      e = launch_prep_copies(a.dout, a.dosb, a.dosh, a.dosl, a.B, a.Hq, a.Lq, D, a.dor, nullptr, stream);
-    // The dK/dV kernel reads its own key rows from k and v; the row-major
-    // copies serve only the recomputing dQ kernel (no staged dS), the
-    // head_dim-major k copy both dQ kernels.
-    const bool rows = a.ds == nullptr;
-    if (e == hipSuccess)
-      e = launch_prep_copies(a.k, a.ksb, a.ksh, a.ksl, a.B, a.Hkv, a.Lk, D, rows ? a.kr : nullptr, a.kt, stream,
-                             nullptr, a.cos_k, a.sin_k, a.rksb);
-    if (e == hipSuccess && rows)
-      e = launch_prep_copies(a.v, a.vsb, a.vsh, a.vsl, a.B, a.Hkv, a.Lk, D, a.vr, nullptr, stream);
-    if (e == hipSuccess) e = launch_key_prep(a.mask, a.msb, a.B, a.Lk, a.kbias, a.kfull, stream);
-    if (e != hipSuccess) return e;
-  }
-  if (!a.reuse_q) {
-    constexpr int RPB = 256 / (D / 8);
-    const int64_t rows = (int64_t)a.B * a.Hq * a.Lqp;
-    LaunchTimer timer(kKidBwdPre, stream);
-    hipLaunchKernelGGL(bwd_pre_kernel<D>, dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, stream, a);
-  }
+  const hipError_t e = launch_prep_bwd(a, D, stream);
+  if (e != hipSuccess) return e;
   // dK/dV (and, with staged dS, dQ) per pass over (b, kv head) pairs.
   const int nkv_all = a.B * a.Hkv;
   const int step = a.ds ? kv_per_pass : nkv_all;

@@ -148,7 +148,6 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_kernel(FwdArgs a) {
   const u32x4 rb = make_rsrc(a.kbias + (int64_t)b * a.Lkp, (uint32_t)(a.Lkp + 64) * 4);
   // Flags are padded by 64 entries: the 64 read from a tile start stay inside.
   const u32x4 rf = make_rsrc(a.kfull + (int64_t)b * (a.Lkp / 32), (uint32_t)(a.Lkp / 32 + 64) * 4);
-  const int tend = t0 + ntile;  // tiles t0 .. tend-1 (all of them without windows)
 
   using KSt = TileStager<BN, KRL, NW>;  // 64 K rows of D channels
   using VSt = TileStager<D, BN, NW>;  // D V^T rows of 64 keys (row stride Lkp)
@@ -274,14 +273,43 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_kernel(FwdArgs a) {
           qn2 = fmaf(x, x, qn2);
         }
       qn2 = halves_sum(qn2);
-      // Largest squared k row norm of the head: a wave maximum over its tiles.
+      // Largest squared k row norm of the head: a wave maximum over its tiles;
+      // and the range of tiles not marked as contributing nothing.
       const int ntk = a.Lkp / 64;
       const uint32_t* km = a.kmax2 + bhk * ntk;
       float km2 = 0.f;
-      for (int i = lane; i < ntk; i += 64) km2 = fmaxf(km2, __uint_as_float(km[i]));
+      int lo = ntk, hi = 0;
+      for (int i = lane; i < ntk; i += 64) {
+        const uint32_t w = km[i];
+        km2 = fmaxf(km2, __uint_as_float(w & ~kTileSkip));
+        if (!(w & kTileSkip)) {
+          lo = min(lo, i);
+          hi = max(hi, i + 1);
+        }
+      }
 #pragma unroll
       for (int off = 32; off > 0; off >>= 1) km2 = fmaxf(km2, __shfl_xor(km2, off));
       bound = sqrtf(qn2) * sqrtf(km2) * (1.f + 1.f / 1024.f);
+      if constexpr (!WIN) {
+        if (a.mask != nullptr) {
+          // Tiles outside the range are left out where that changes nothing:
+          // their scores are -inf unless a row of q is not finite or a
+          // product overflows, which every row's bound must rule out.
+#pragma unroll
+          for (int off = 32; off > 0; off >>= 1) {
+            lo = min(lo, __shfl_xor(lo, off));
+            hi = max(hi, __shfl_xor(hi, off));
+          }
+          lo = __builtin_amdgcn_readfirstlane(lo);
+          hi = __builtin_amdgcn_readfirstlane(hi);
+          if (lo > 0 || hi < ntile) {  // the same for every wave
+            if (__syncthreads_and(bound <= 3.0e38f)) {
+              t0 = lo < hi ? lo : 0;
+              ntile = hi - t0;
+            }
+          }
+        }
+      }
     }
   }
   int bounded = 0;  // wave-uniform
@@ -516,9 +544,9 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_kernel(FwdArgs a) {
     for (int i = done; i < kStageOps; ++i) stage_op(t, nextc, i);
   };
 
+  const int tend = t0 + ntile;  // tiles t0 .. tend-1
   retire_prologue_loads();
-  // ntile is the same for every wave of the workgroup (0: every row's window
-  // is empty, nothing to visit).
+  // ntile is the same for every wave of the workgroup (0: no key to visit).
   if (ntile > 0) {
     {
       using B0 = std::integral_constant<int, 0>;
@@ -709,17 +737,12 @@ __global__ void attn_empty_kernel(bf16* o, int64_t osb, int64_t osh, int64_t osl
 template <int D>
 static hipError_t launch_fwd_d(const FwdArgs& a, hipStream_t stream) {
   const bool fp8 = a.k8 != nullptr;
-  {
+  hipError_t e = launch_prep_fwd(a, D, stream);
+  if (e == hipSuccess && fp8) {
     LaunchTimer timer(kKidTranspose, stream);
-    hipError_t e = launch_key_prep(a.mask, a.msb, a.B, a.Lk, a.kbias, a.kfull, stream);
-    if (e == hipSuccess)
-      e = fp8 ? launch_quantize_rows(a.k, a.ksb, a.ksh, a.ksl, a.B, a.Hkv, a.Lk, D, a.k_scale, a.k8, a.kmax2,
-                                     stream)
-              : launch_prep_copies(a.k, a.ksb, a.ksh, a.ksl, a.B, a.Hkv, a.Lk, D, a.kr, nullptr, stream, a.kmax2,
-                                   a.cos_k, a.sin_k, a.rksb);
-    if (e == hipSuccess) e = launch_prep_copies(a.v, a.vsb, a.vsh, a.vsl, a.B, a.Hkv, a.Lk, D, nullptr, a.vt, stream);
-    if (e != hipSuccess) return e;
+    e = launch_quantize_rows(a.k, a.ksb, a.ksh, a.ksl, a.B, a.Hkv, a.Lk, D, a.k_scale, a.k8, a.kmax2, stream);
   }
+  if (e != hipSuccess) return e;
   const int nqt = (a.Lq + 255) / 256;
   const dim3 grid(nqt * a.B * a.Hq);
   const dim3 block(512);

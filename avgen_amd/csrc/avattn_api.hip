@@ -131,6 +131,15 @@ BwdWorkspace bwd_workspace(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lq, int32
   return w;
 }
 
+// BwdArgs::khull and kskip of a backward with staged dS and no windows: they
+// take the place of the K row copy, which only the recomputing dQ kernel
+// reads (8 KB or more per 64-key tile, against 12 bytes).
+void set_hull(BwdArgs& a, char* ws, const BwdWorkspace& w) {
+  if (a.wlo) return;
+  a.khull = reinterpret_cast<int*>(ws + w.kr);
+  a.kskip = a.mask ? a.khull + 2 * (size_t)a.nkv : nullptr;
+}
+
 // Key windows: both arrays or neither, 4-byte aligned, batch stride 0
 // (shared) or >= len_q; not with the fused RoPE or fp8 variants.
 int check_windows(const int32_t* lo, const int32_t* hi, int64_t batch_stride, int32_t len_q, bool excluded) {
@@ -524,6 +533,7 @@ static int bwd_impl(const void* dout, const void* q, const void* k, const void* 
     const size_t npass = ((size_t)a.nkv + fit - 1) / fit;
     kv_per_pass = (int)(((size_t)a.nkv + npass - 1) / npass);
     a.ds = reinterpret_cast<bf16*>(ws + off);
+    set_hull(a, ws, wl);
   }
   return launch_status(launch_bwd(a, head_dim, kv_per_pass, s));
 }
@@ -612,6 +622,7 @@ int avattn_bwd_dq_staged(int32_t batch, int32_t heads_q, int32_t heads_kv, int32
   a.kv0 = 0;
   a.nkv = batch * heads_kv;
   a.ds = reinterpret_cast<bf16*>(ws + off);
+  set_hull(a, ws, wl);
   return launch_status(launch_bwd_dq_staged(a, head_dim, s));
 }
 

@@ -9,6 +9,9 @@
 
 namespace avattn {
 
+// Mark in the sign bit of a kmax2 entry (see FwdArgs).
+constexpr uint32_t kTileSkip = 0x80000000u;
+
 struct FwdArgs {
   const bf16* q;
   const bf16* k;
@@ -45,7 +48,9 @@ struct FwdArgs {
   // Largest squared row norm of k (bf16 path) or of k8 in e4m3 units (fp8)
   // per 64-key tile, (b, kv head, tile) at ((b*Hkv + h)*(Lkp/64) + tile),
   // float bits (written by the k copy): the largest over a head bounds every
-  // score of a query row by |q_row| * sqrt(max).
+  // score of a query row by |q_row| * sqrt(max).  The sign bit (kTileSkip,
+  // bf16 path with a mask only) marks a tile that contributes nothing: no
+  // key of it is attended and its k and v are finite.
   uint32_t* kmax2;
   // Key windows (null: every key): query row i of batch b attends to keys
   // [wlo[b*wsb + i], whi[b*wsb + i]) (and the key mask), shared by all heads.
@@ -114,6 +119,13 @@ struct BwdArgs {
   float* kbias;  // (B, Lkp): 0 attended / -inf
   int* kfull;    // (B, Lkp/32): 1 if every key of the 32-key tile is attended
   int Lqp, Lkp;
+  // Staged dS without windows: khull[2 p], khull[2 p + 1] bound the 64-key
+  // tiles of pair p = b*Hkv + hk that can contribute; outside them no key is
+  // attended and k is finite, so dS is exactly 0 there: the dK/dV kernel does
+  // not form it, the dQ kernel does not read it.  kskip: per (p, tile), the
+  // marks it is made from (null without a mask).
+  int* khull;
+  int* kskip;
   // dq as an fp32 accumulator (dq_acc += this chunk's dq; dq is then null),
   // strides dqsb/dqsh/dqsl in floats.
   float* dq_acc;
@@ -256,20 +268,12 @@ class LaunchTimer {
 // padded length; validated problems fit in int.
 inline int64_t transpose_padded_len(int64_t L) { return (L + 63) / 64 * 64; }
 
-// Padded key bias (B, Lkp) floats (0 attended / -inf) and per-32-key-tile
-// "all attended" flags (B, Lkp/32); mask may be null (only the tail is masked).
-hipError_t launch_key_prep(const uint8_t* mask, int64_t msb, int B, int Lk, float* kbias, int* kfull,
-                           hipStream_t stream);
-
-// x (B, H, L, D) strided -> xr (B*H, Lp, D) and/or xt (B*H, D, Lp), contiguous,
-// zero padded to Lp = transpose_padded_len(L); either output may be null.
-// With rowmax2 set (B*H*(Lp/64) words), also the largest squared row norm of
-// each 64-row tile of each (b, h) slice, as float bits.
-// With cos/sin tables (b, 0, i, pair) at b*tsb + i*(D/2) + pair, rows are
-// rotated (rotate8) before they are copied.
-hipError_t launch_prep_copies(const bf16* x, int64_t sb, int64_t sh, int64_t sl, int B, int H, int L, int D,
-                              bf16* xr, bf16* xt, hipStream_t stream, uint32_t* rowmax2 = nullptr,
-                              const float* cos_t = nullptr, const float* sin_t = nullptr, int64_t tsb = 0);
+// The forward's preparation (FwdArgs::kr, vt, kbias, kfull, kmax2; with k8
+// set everything but the K copy and kmax2).
+hipError_t launch_prep_fwd(const FwdArgs& a, int head_dim, hipStream_t stream);
+// The backward's (BwdArgs::kt, kbias, kfull, khull, the row copies it needs
+// and, unless a.reuse_q, lse2 and ndelta).
+hipError_t launch_prep_bwd(const BwdArgs& a, int head_dim, hipStream_t stream);
 
 // dq (bf16, strided) = transposed rotation of bf16(dq_acc) (fp32, strided);
 // a plain cast when cos_t is null.

@@ -19,32 +19,28 @@
 
 namespace avattn {
 
-// One workgroup copies 64 sequence rows x D channels of one (b, h), rotating
-// each row first when rotation tables are given (the copies then hold the
-// rotated rows src/avgen/models/rope.py:332-338 produces).  With
-// rowmax2 set, it also writes the largest squared norm of its (valid) rows to
-// rowmax2[(b*H + h)*(Lp/64) + tile] as float bits (one plain store per
-// workgroup; an atomic per wave into one word per head serialised badly).
-template <int D>
-__global__ __launch_bounds__(256) void prep_copies_kernel(const bf16* __restrict__ x, int64_t sb, int64_t sh,
-                                                          int64_t sl, int H, int L, int Lp, bf16* __restrict__ xr,
-                                                          bf16* __restrict__ xt, uint32_t* __restrict__ rowmax2,
-                                                          const float* __restrict__ ct, const float* __restrict__ st,
-                                                          int64_t tsb) {
-  constexpr int S = 64;       // sequence rows per workgroup
+// One 64-row tile of x (256 threads): rows s0 .. s0 + 63 of one (b, h) slice
+// whose row 0 is at `src`, rotated first when the slice's tables are given
+// (the copies then hold the rotated rows src/avgen/models/rope.py:332-338
+// produces), to `xr` (row-major, D apart) and / or `xt` (head_dim-major, Lp
+// apart; both already at the tile).  Returns the thread's share of the
+// largest squared row norm (NORM) and of "every value is finite" (FINITE).
+struct TileScan {
+  float nmax;
+  bool finite;
+};
+template <int D, bool NORM>
+__device__ __forceinline__ TileScan copy_tile(const bf16* __restrict__ src, int64_t sl, int s0, int L, int Lp,
+                                              bf16* __restrict__ xr, bf16* __restrict__ xt,
+                                              const float* __restrict__ ct, const float* __restrict__ st,
+                                              bool check_finite, bf16* tile) {
+  constexpr int S = 64;       // sequence rows per tile
   constexpr int CPR = D / 8;  // 16-byte chunks per row
   constexpr int LD = D + 2;   // LDS row pitch in bf16 (odd word count: column reads spread over banks)
-  __shared__ bf16 tile[S * LD];
   const int tid = threadIdx.x;
-  const int ntiles = Lp / S;
-  const int s0 = (blockIdx.x % ntiles) * S;
-  const int bh = blockIdx.x / ntiles;
-  const int b = bh / H, h = bh % H;
-  const bf16* src = x + b * sb + h * sh;
-
+  TileScan r{0.f, true};
   // Load 64 rows (zeros past L) as 16-byte chunks; write the row-major copy
   // and scatter into the pitched tile for the head_dim-major one.
-  float nmax = 0.f;  // largest squared row norm seen by this thread's rows
 #pragma unroll
   for (int i = 0; i < S * CPR / 256; ++i) {
     const int c = tid + i * 256;
@@ -54,95 +50,276 @@ __global__ __launch_bounds__(256) void prep_copies_kernel(const bf16* __restrict
       v = *reinterpret_cast<const u32x4*>(src + (int64_t)(s0 + row) * sl + ch * 8);
       if (ct) {
         // Channels 8*ch .. +7 are pairs 4*ch .. +3 of row s0 + row.
-        const int64_t t = b * tsb + (int64_t)(s0 + row) * (D / 2) + 4 * ch;
+        const int64_t t = (int64_t)(s0 + row) * (D / 2) + 4 * ch;
         v = rotate8(v, *reinterpret_cast<const f32x4*>(ct + t), *reinterpret_cast<const f32x4*>(st + t), false);
       }
     }
-    if (xr) *reinterpret_cast<u32x4*>(xr + ((int64_t)bh * Lp + s0 + row) * D + ch * 8) = v;
-    uint32_t* dst = reinterpret_cast<uint32_t*>(tile + row * LD + ch * 8);
+    if (check_finite) {
 #pragma unroll
-    for (int w = 0; w < 4; ++w) dst[w] = v[w];
-    if (rowmax2) {
+      for (int w = 0; w < 4; ++w)
+        r.finite = r.finite && (v[w] & 0x7f80u) != 0x7f80u && (v[w] & 0x7f800000u) != 0x7f800000u;
+    }
+    if (xr) *reinterpret_cast<u32x4*>(xr + row * D + ch * 8) = v;
+    if (xt) {
+      uint32_t* dst = reinterpret_cast<uint32_t*>(tile + row * LD + ch * 8);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) dst[w] = v[w];
+    }
+    if constexpr (NORM) {
       // A row's CPR chunks sit in CPR consecutive lanes: sum their squares.
       float n = 0.f;
 #pragma unroll
       for (int w = 0; w < 4; ++w) n = fmaf(bf16_lo(v[w]), bf16_lo(v[w]), fmaf(bf16_hi(v[w]), bf16_hi(v[w]), n));
 #pragma unroll
       for (int off = 1; off < CPR; off <<= 1) n += __shfl_xor(n, off);
-      nmax = fmaxf(nmax, n);
+      r.nmax = fmaxf(r.nmax, n);
     }
   }
-  if (rowmax2) {
-    __shared__ float wmax[4];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) nmax = fmaxf(nmax, __shfl_xor(nmax, off));
-    if ((tid & 63) == 0) wmax[tid >> 6] = nmax;
+  if (xt) {
     __syncthreads();
-    if (tid == 0) rowmax2[blockIdx.x] = __float_as_uint(fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])));
-  }
-  if (!xt) return;
-  __syncthreads();
-
-  // Each thread writes 16-byte chunks of head_dim-major rows: 8 consecutive
-  // sequence positions of one channel.
-  bf16* dst = xt + (int64_t)bh * D * Lp + s0;
+    // Each thread writes 16-byte chunks of head_dim-major rows: 8 consecutive
+    // sequence positions of one channel.
 #pragma unroll
-  for (int i = 0; i < D * (S / 8) / 256; ++i) {
-    const int c = tid + i * 256;
-    const int d = c / (S / 8), j = c % (S / 8);
-    u32x4 v;
+    for (int i = 0; i < D * (S / 8) / 256; ++i) {
+      const int c = tid + i * 256;
+      const int d = c / (S / 8), j = c % (S / 8);
+      u32x4 v;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const uint16_t lo = __builtin_bit_cast(uint16_t, tile[(8 * j + 2 * w) * LD + d]);
+        const uint16_t hi = __builtin_bit_cast(uint16_t, tile[(8 * j + 2 * w + 1) * LD + d]);
+        v[w] = (uint32_t)lo | ((uint32_t)hi << 16);
+      }
+      *reinterpret_cast<u32x4*>(xt + (int64_t)d * Lp + 8 * j) = v;
+    }
+  }
+  return r;
+}
+
+// Whether every value of a 64-row tile is finite (this thread's share).
+template <int D>
+__device__ __forceinline__ bool tile_finite(const bf16* __restrict__ src, int64_t sl, int s0, int L) {
+  constexpr int CPR = D / 8;
+  bool ok = true;
+#pragma unroll
+  for (int i = 0; i < 64 * CPR / 256; ++i) {
+    const int c = threadIdx.x + i * 256;
+    const int row = s0 + c / CPR;
+    if (row < L) {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(src + (int64_t)row * sl + (c % CPR) * 8);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) ok = ok && (v[w] & 0x7f80u) != 0x7f80u && (v[w] & 0x7f800000u) != 0x7f800000u;
+    }
+  }
+  return ok;
+}
+
+// The 64 lanes of a wave as the keys j0 .. j0 + 63 of batch b: which are
+// attended (j < Lk and the mask, if any, is nonzero).
+__device__ __forceinline__ uint64_t attended_keys(const uint8_t* mask, int64_t msb, int b, int j0, int Lk) {
+  const int j = j0 + (threadIdx.x & 63);
+  return __builtin_amdgcn_ballot_w64(j < Lk && (mask == nullptr || mask[b * msb + j] != 0));
+}
+
+// Key bias and flags of one 64-key tile (threads 0..63): kbias[b*Lkp + j] = 0
+// if key j is attended, else -inf; kfull[b*(Lkp/32) + t] = 1 if all 32 keys
+// of tile t are attended.
+__device__ __forceinline__ void write_key_bias(uint64_t att, int b, int j0, int Lkp, float* __restrict__ kbias,
+                                               int* __restrict__ kfull) {
+  const int lane = threadIdx.x;
+  if (lane >= 64) return;
+  kbias[(int64_t)b * Lkp + j0 + lane] = (att >> lane) & 1 ? 0.f : kNegInf;
+  if (lane < 2) kfull[(int64_t)b * (Lkp / 32) + j0 / 32 + lane] = (uint32_t)(att >> (32 * lane)) == 0xffffffffu;
+}
+
+// Forward preparation, one launch (separate ones cost 4-8 us each at short
+// sequences: K, V and key-bias launches 39 us of a 338 us call at
+// (2,20,3600,128)).  Workgroups [0, nk): K row copy of one 64-key tile of one
+// (b, kv head) with the tile's largest squared row norm in kmax2 (none with
+// fp8, whose K copy is launch_quantize_rows); then the V^T copy of one tile
+// each, those of kv head 0 also writing the tile's key bias and flags.  A
+// tile without an attended key whose k and v are finite is marked in the sign
+// bit of its kmax2 (the norm itself is >= 0): it contributes exactly nothing
+// and the forward may leave it out.  Leaving such tiles out at both ends here
+// and in the backward took 75,600 queries x 512 text keys (one sample of 388
+// keys, one of none, 40 heads, D 128, fwd+bwd) from 7.35 to 5.59 ms.
+template <int D>
+__global__ __launch_bounds__(256) void prep_fwd_kernel(FwdArgs a, int nk) {
+  __shared__ bf16 tile[64 * (D + 2)];
+  __shared__ float wmax[4];
+  __shared__ int wfin[4];
+  const int nt = a.Lkp / 64;
+  const bool is_k = (int)blockIdx.x < nk;
+  const int u = is_k ? blockIdx.x : blockIdx.x - nk;
+  const int t = u % nt, bh = u / nt;
+  const int b = bh / a.Hkv, h = bh % a.Hkv;
+  const int s0 = 64 * t;
+  if (is_k) {
+    const bool unattended = a.mask != nullptr && attended_keys(a.mask, a.msb, b, s0, a.Lk) == 0;
+    const float* ct = a.cos_k ? a.cos_k + b * a.rksb : nullptr;
+    const float* st = a.cos_k ? a.sin_k + b * a.rksb : nullptr;
+    TileScan r = copy_tile<D, true>(a.k + b * a.ksb + h * a.ksh, a.ksl, s0, a.Lk, a.Lkp,
+                                    a.kr + ((int64_t)bh * a.Lkp + s0) * D, nullptr, ct, st, unattended, tile);
+    if (unattended) r.finite = r.finite && tile_finite<D>(a.v + b * a.vsb + h * a.vsh, a.vsl, s0, a.Lk);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) r.nmax = fmaxf(r.nmax, __shfl_xor(r.nmax, off));
+    const int fin = __all(r.finite);
+    if ((threadIdx.x & 63) == 0) {
+      wmax[threadIdx.x >> 6] = r.nmax;
+      wfin[threadIdx.x >> 6] = fin;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const bool skip = unattended && wfin[0] && wfin[1] && wfin[2] && wfin[3];
+      a.kmax2[(int64_t)bh * nt + t] = __float_as_uint(fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]))) |
+                                      (skip ? kTileSkip : 0u);
+    }
+  } else {
+    if (h == 0) write_key_bias(attended_keys(a.mask, a.msb, b, s0, a.Lk), b, s0, a.Lkp, a.kbias, a.kfull);
+    copy_tile<D, false>(a.v + b * a.vsb + h * a.vsh, a.vsl, s0, a.Lk, a.Lkp, nullptr,
+                        a.vt + (int64_t)bh * D * a.Lkp + s0, nullptr, nullptr, false, tile);
+  }
+}
+
+// Backward preparation, one launch.  Workgroups in order: one 64-key tile of
+// one (b, kv head) each (K^T copy, and without staged dS the K and V row
+// copies; those of kv head 0 write the tile's key bias and flags; with a mask
+// and staged dS, kskip says whether no key of the tile is attended while its
+// k is finite, see key_hull_kernel); then, unless the query side is reused,
+// one 64-row tile of one (b, query head) each for the q and dO copies the
+// dK/dV kernel needs, and the row statistics: lse2 = lse * log2(e) (+inf for
+// -inf and padded rows, whose P is then exactly 0) and ndelta =
+// -rowsum(dout * out), RPB rows per workgroup.  Under a mask a row with lse
+// -inf attends nothing: its dout and out are not read.
+template <int D>
+__global__ __launch_bounds__(256) void prep_bwd_kernel(BwdArgs a, int nk, int nq, int nd) {
+  __shared__ bf16 tile[64 * (D + 2)];
+  int u = blockIdx.x;
+  if (u < nk) {
+    const int nt = a.Lkp / 64;
+    const int t = u % nt, bh = u / nt;
+    const int b = bh / a.Hkv, h = bh % a.Hkv;
+    const int s0 = 64 * t;
+    const uint64_t att = attended_keys(a.mask, a.msb, b, s0, a.Lk);
+    if (h == 0) write_key_bias(att, b, s0, a.Lkp, a.kbias, a.kfull);
+    const float* ct = a.cos_k ? a.cos_k + b * a.rksb : nullptr;
+    const float* st = a.cos_k ? a.sin_k + b * a.rksb : nullptr;
+    const bool rows = a.ds == nullptr;
+    const int64_t row0 = ((int64_t)bh * a.Lkp + s0) * D;
+    const bool scan = a.kskip != nullptr && att == 0;
+    const TileScan r = copy_tile<D, false>(a.k + b * a.ksb + h * a.ksh, a.ksl, s0, a.Lk, a.Lkp,
+                                           rows ? a.kr + row0 : nullptr, a.kt + (int64_t)bh * D * a.Lkp + s0, ct, st,
+                                           scan, tile);
+    if (rows)
+      copy_tile<D, false>(a.v + b * a.vsb + h * a.vsh, a.vsl, s0, a.Lk, a.Lkp, a.vr + row0, nullptr, nullptr,
+                          nullptr, false, tile);
+    if (a.kskip != nullptr) {
+      const int skip = __syncthreads_and(scan && r.finite);
+      if (threadIdx.x == 0) a.kskip[(int64_t)bh * nt + t] = skip;
+    } else if (a.khull != nullptr && t == 0 && threadIdx.x == 0) {
+      a.khull[2 * bh] = 0;
+      a.khull[2 * bh + 1] = nt;
+    }
+    return;
+  }
+  u -= nk;
+  if (u < nq + nd) {
+    const bool is_q = u < nq;
+    if (!is_q) u -= nq;
+    const int nt = a.Lqp / 64;
+    const int t = u % nt, bh = u / nt;
+    const int b = bh / a.Hq, h = bh % a.Hq;
+    const int64_t row0 = ((int64_t)bh * a.Lqp + 64 * t) * D;
+    if (is_q)
+      copy_tile<D, false>(a.q + b * a.qsb + h * a.qsh, a.qsl, 64 * t, a.Lq, a.Lqp, a.qr + row0, nullptr,
+                          a.cos_q ? a.cos_q + b * a.rqsb : nullptr, a.cos_q ? a.sin_q + b * a.rqsb : nullptr, false,
+                          tile);
+    else
+      copy_tile<D, false>(a.dout + b * a.dosb + h * a.dosh, a.dosl, 64 * t, a.Lq, a.Lqp, a.dor + row0, nullptr,
+                          nullptr, nullptr, false, tile);
+    return;
+  }
+  u -= nq + nd;
+  constexpr int TPR = D / 8;  // threads per row
+  constexpr int RPB = 256 / TPR;
+  const int64_t rows = (int64_t)a.B * a.Hq * a.Lqp;
+  const int64_t row = (int64_t)u * RPB + threadIdx.x / TPR;
+  const int c = threadIdx.x % TPR;
+  const int i = (int)(row % a.Lqp);
+  const int64_t bh = row / a.Lqp;
+  const bool valid = row < rows && i < a.Lq;
+  const float l = valid ? a.lse[bh * a.Lq + i] : kNegInf;
+  float acc = 0.f;
+  if (valid && (a.mask == nullptr || l != kNegInf)) {
+    const int h = (int)(bh % a.Hq);
+    const int b = (int)(bh / a.Hq);
+    const u32x4 x = *reinterpret_cast<const u32x4*>(a.dout + b * a.dosb + h * a.dosh + (int64_t)i * a.dosl + 8 * c);
+    const u32x4 y = *reinterpret_cast<const u32x4*>(a.out + b * a.osb + h * a.osh + (int64_t)i * a.osl + 8 * c);
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-      const uint16_t lo = __builtin_bit_cast(uint16_t, tile[(8 * j + 2 * w) * LD + d]);
-      const uint16_t hi = __builtin_bit_cast(uint16_t, tile[(8 * j + 2 * w + 1) * LD + d]);
-      v[w] = (uint32_t)lo | ((uint32_t)hi << 16);
+      acc = fmaf(__uint_as_float(x[w] << 16), __uint_as_float(y[w] << 16), acc);
+      acc = fmaf(__uint_as_float(x[w] & 0xffff0000u), __uint_as_float(y[w] & 0xffff0000u), acc);
     }
-    *reinterpret_cast<u32x4*>(dst + (int64_t)d * Lp + 8 * j) = v;
+  }
+#pragma unroll
+  for (int off = TPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, TPR);
+  if (row < rows && c == 0) {
+    a.ndelta[row] = -acc;
+    a.lse2[row] = (l == kNegInf) ? kPosInf : l * kLog2e;
   }
 }
 
-// Key bias and tile flags: kbias[b*Lkp + j] = 0 if key j < Lk is attended
-// (mask nonzero, or no mask) else -inf, for j < Lkp; kfull[b*(Lkp/32) + t] = 1
-// if all 32 keys of tile t are attended.  One thread per 32-key tile.
-__global__ __launch_bounds__(256) void key_prep_kernel(const uint8_t* __restrict__ mask, int64_t msb, int B, int Lk,
-                                                       int Lkp, float* __restrict__ kbias, int* __restrict__ kfull) {
-  const int tiles = Lkp / 32;
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)B * tiles) return;
-  const int b = (int)(t / tiles), j0 = (int)(t % tiles) * 32;
-  int all = 1;
-  for (int j = j0; j < j0 + 32; ++j) {
-    const bool valid = j < Lk && (mask == nullptr || mask[b * msb + j] != 0);
-    kbias[(int64_t)b * Lkp + j] = valid ? 0.f : kNegInf;
-    all &= valid ? 1 : 0;
+// Per (b, kv head), the range [khull[2 p], khull[2 p + 1]) of 64-key tiles
+// outside which every tile is marked in kskip (empty when all are).  One wave
+// per pair.
+__global__ __launch_bounds__(64) void key_hull_kernel(const int* __restrict__ kskip, int nt, int* __restrict__ khull) {
+  int lo = nt, hi = 0;
+  for (int t = threadIdx.x; t < nt; t += 64) {
+    if (kskip[(int64_t)blockIdx.x * nt + t] == 0) {
+      lo = min(lo, t);
+      hi = max(hi, t + 1);
+    }
   }
-  kfull[t] = all;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    lo = min(lo, __shfl_xor(lo, off));
+    hi = max(hi, __shfl_xor(hi, off));
+  }
+  if (threadIdx.x == 0) {
+    khull[2 * blockIdx.x] = lo < hi ? lo : 0;
+    khull[2 * blockIdx.x + 1] = hi;
+  }
 }
 
-hipError_t launch_key_prep(const uint8_t* mask, int64_t msb, int B, int Lk, float* kbias, int* kfull,
-                           hipStream_t stream) {
-  const int Lkp = transpose_padded_len(Lk);
-  const int64_t n = (int64_t)B * (Lkp / 32);
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(key_prep_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, mask, msb, B, Lk, Lkp,
-                     kbias, kfull);
+hipError_t launch_prep_fwd(const FwdArgs& a, int head_dim, hipStream_t stream) {
+  const int64_t tiles = (int64_t)a.B * a.Hkv * (a.Lkp / 64);
+  if (2 * tiles > 2147483647) return hipErrorInvalidValue;
+  const int nk = a.k8 ? 0 : (int)tiles;
+  const dim3 grid((unsigned)(nk + tiles));
+  LaunchTimer timer(kKidTranspose, stream);
+  if (head_dim == 128)
+    hipLaunchKernelGGL(prep_fwd_kernel<128>, grid, dim3(256), 0, stream, a, nk);
+  else
+    hipLaunchKernelGGL(prep_fwd_kernel<64>, grid, dim3(256), 0, stream, a, nk);
   return hipGetLastError();
 }
 
-hipError_t launch_prep_copies(const bf16* x, int64_t sb, int64_t sh, int64_t sl, int B, int H, int L, int D,
-                              bf16* xr, bf16* xt, hipStream_t stream, uint32_t* rowmax2, const float* cos_t,
-                              const float* sin_t, int64_t tsb) {
-  const int Lp = transpose_padded_len(L);
-  if ((int64_t)B * H == 0 || Lp == 0 || (!xr && !xt)) return hipSuccess;
-  const int64_t blocks = (int64_t)(Lp / 64) * B * H;
-  if (blocks > 2147483647) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)blocks);
-  if (D == 128)
-    hipLaunchKernelGGL(prep_copies_kernel<128>, grid, dim3(256), 0, stream, x, sb, sh, sl, H, L, Lp, xr, xt, rowmax2,
-                       cos_t, sin_t, tsb);
+hipError_t launch_prep_bwd(const BwdArgs& a, int head_dim, hipStream_t stream) {
+  const int64_t nk = (int64_t)a.B * a.Hkv * (a.Lkp / 64);
+  const int64_t qtiles = (int64_t)a.B * a.Hq * (a.Lqp / 64);
+  const int64_t nq = !a.reuse_q && a.qt == a.qr ? qtiles : 0, nd = !a.reuse_q && a.dt == a.dor ? qtiles : 0;
+  const int rpb = 256 / (head_dim / 8);
+  const int64_t ns = a.reuse_q ? 0 : ((int64_t)a.B * a.Hq * a.Lqp + rpb - 1) / rpb;
+  if (nk + nq + nd + ns > 2147483647) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(nk + nq + nd + ns));
+  LaunchTimer timer(kKidBwdPre, stream);
+  if (head_dim == 128)
+    hipLaunchKernelGGL(prep_bwd_kernel<128>, grid, dim3(256), 0, stream, a, (int)nk, (int)nq, (int)nd);
   else
-    hipLaunchKernelGGL(prep_copies_kernel<64>, grid, dim3(256), 0, stream, x, sb, sh, sl, H, L, Lp, xr, xt, rowmax2,
-                       cos_t, sin_t, tsb);
+    hipLaunchKernelGGL(prep_bwd_kernel<64>, grid, dim3(256), 0, stream, a, (int)nk, (int)nq, (int)nd);
+  if (a.kskip != nullptr)
+    hipLaunchKernelGGL(key_hull_kernel, dim3((unsigned)(a.B * a.Hkv)), dim3(64), 0, stream, a.kskip, a.Lkp / 64,
+                       a.khull);
   return hipGetLastError();
 }
 
