@@ -1276,7 +1276,8 @@ __global__ __launch_bounds__(512, 1) void bwd_dq_ds_kernel(BwdArgs a) {
   }
   wait_vmem();  // the last (re-staged) loads
 
-  if (qvalid && a.dq_acc) {
+  if (a.dq_acc) {
+    if (!qvalid) return;
     float* op = a.dq_acc + b * a.dqsb + h * a.dqsh + (int64_t)qrow * a.dqsl;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -1288,8 +1289,12 @@ __global__ __launch_bounds__(512, 1) void bwd_dq_ds_kernel(BwdArgs a) {
         for (int r = 0; r < 4; ++r) w[r] += acc[dt][4 * g + r] * a.scale;
         *p = w;
       }
-  } else if (qvalid) {
-    bf16* op = a.dq + b * a.dqsb + h * a.dqsh + (int64_t)qrow * a.dqsl;
+  } else if (a.dq) {
+    // bf16 rows leave through LDS (no stage is read any more), whole rows per
+    // store instruction (see the forward's epilogue).
+    barrier_lds();
+    bf16* ep = reinterpret_cast<bf16*>(st) + wave * 32 * D;
+    static_assert(sizeof(st) >= NW * 32 * D * sizeof(bf16), "the output rows fit the stages");
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -1297,8 +1302,17 @@ __global__ __launch_bounds__(512, 1) void bwd_dq_ds_kernel(BwdArgs a) {
         u32x2 w;
         w[0] = pack_bf16x2(acc[dt][4 * g] * a.scale, acc[dt][4 * g + 1] * a.scale);
         w[1] = pack_bf16x2(acc[dt][4 * g + 2] * a.scale, acc[dt][4 * g + 3] * a.scale);
-        *reinterpret_cast<u32x2*>(op + dt * 32 + 8 * g + 4 * hh) = w;
+        *reinterpret_cast<u32x2*>(ep + TileLayout<D>::off(l32, dt * 32 + 8 * g) + 4 * hh) = w;
       }
+    constexpr int kCpr = D / 8, kRpi = 64 / kCpr;  // chunks per row, rows per store
+    const int er = lane / kCpr, ec = 8 * (lane % kCpr);
+    bf16* op = a.dq + b * a.dqsb + h * a.dqsh + ec;
+#pragma unroll
+    for (int i = 0; i < 32 / kRpi; ++i) {
+      const int r = i * kRpi + er, row = qg * 32 + r;
+      const u32x4 x = *reinterpret_cast<const u32x4*>(ep + TileLayout<D>::off(r, ec));
+      if (row < a.Lq) *reinterpret_cast<u32x4*>(op + (int64_t)row * a.dqsl) = x;
+    }
   }
 }
 
