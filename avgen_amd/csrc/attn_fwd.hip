@@ -47,15 +47,22 @@ namespace avattn {
 // accumulator starts from -m.  K comes from the e4m3 copy (fp8.hip).  P, V
 // and O^T += V^T P^T stay bf16 / fp32 as above.
 //
+// SMALL: workgroups of 128 query rows and 4 waves, two LDS stages, two
+// workgroups per CU (three at D 64): the two waves of a SIMD belong to
+// different workgroups, so one's loads, prologue and output overlap the
+// other's products without the staggered order.  Each wave runs QK^T(t),
+// softmax(t), PV(t), with tile t + 1 loaded meanwhile.  See use_small.
+//
 // WIN: per-query-row key windows [wlo, whi) (FwdArgs::wlo/whi).  The
 // workgroup visits only the tiles that meet the union of its rows' windows,
 // and a tile half that is not inside every window of the wave masks each
 // score outside its row's window to -inf (before the key bias and softmax).
-template <int D, bool ROPE, bool FP8, bool WIN>
-__global__ __launch_bounds__(512, 1) void attn_fwd_kernel(FwdArgs a) {
+template <int D, bool ROPE, bool FP8, bool WIN, bool SMALL>
+__global__ __launch_bounds__(SMALL ? 256 : 512, SMALL ? 2 : 1) void attn_fwd_kernel(FwdArgs a) {
   static_assert(!(ROPE && FP8), "the fp8 variant takes rotated q");
   static_assert(!(WIN && FP8), "windows on the bf16 path only");
-  constexpr int NW = 8, BM = 32 * NW, BN = 64;
+  static_assert(!(SMALL && FP8), "small workgroups on the bf16 path only");
+  constexpr int NW = SMALL ? 4 : 8, BM = 32 * NW, BN = 64;
   // k-steps of q k^T: 16 bf16 channels (32x32x16 bf16) or 64 fp8 channels
   // (32x32x64 e4m3) per MFMA.
   constexpr int KS = FP8 ? D / 64 : D / 16;
@@ -109,9 +116,17 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_kernel(FwdArgs a) {
       whi = min(max(a.whi[b * a.wsb + qrow], wlo), a.Lk);
       mlo = wlo;
       mhi = whi;
-      if (wlo < whi) {
-        rlo = wlo;
-        rhi = whi;
+    }
+    // The range is that of the aligned 256 rows around this workgroup's in
+    // both workgroup sizes: which rows a NaN key reaches through 0 x NaN does
+    // not depend on the size chosen.
+    const int urow = qt * BM / 256 * 256 + (SMALL ? tid : wave * 32 + l32);
+    if (urow < a.Lq) {
+      const int ulo = min(max(a.wlo[b * a.wsb + urow], 0), a.Lk);
+      const int uhi = min(max(a.whi[b * a.wsb + urow], ulo), a.Lk);
+      if (ulo < uhi) {
+        rlo = ulo;
+        rhi = uhi;
       }
     }
 #pragma unroll
@@ -531,7 +546,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_kernel(FwdArgs a) {
   // issues exactly kStageOps loads per iteration: the counted waits rely on
   // it.  The fp8 q k^T has only 4 MFMAs per tile, so there the loads ride on
   // PV.
-  constexpr int kLoad0 = 2, kLoadStep = 3;
+  constexpr int kLoad0 = 2, kLoadStep = SMALL ? 1 : 3;
   auto loads_in = [&](int t, auto nextc) __attribute__((always_inline)) {
     return [&, t, nextc](int j) __attribute__((always_inline)) {
       if (j >= kLoad0 && (j - kLoad0) % kLoadStep == 0 && (j - kLoad0) / kLoadStep < kStageOps)
@@ -547,7 +562,33 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_kernel(FwdArgs a) {
   const int tend = t0 + ntile;  // tiles t0 .. tend-1
   retire_prologue_loads();
   // ntile is the same for every wave of the workgroup (0: no key to visit).
-  if (ntile > 0) {
+  if (SMALL && ntile > 0) {
+    using B0 = std::integral_constant<int, 0>;
+    using B1 = std::integral_constant<int, 1>;
+    f32x16 sh[2];
+    bf16x8 pf[2][2];
+#pragma unroll
+    for (int i = 0; i < kStageOps; ++i) stage_op(t0, B0(), i);
+    auto body = [&](int t, auto bufc) __attribute__((always_inline)) {
+      using Next = std::integral_constant<int, 1 - decltype(bufc)::value>;
+      wait_vmem_n<0>();  // tile t landed ...
+      barrier_lds();     // ... for every wave, and tile t - 1's stage is free
+      const Stage& sg = stage_ref(bufc);
+      const int tl = min(t + 1, tend - 1);
+      __builtin_amdgcn_s_setprio(2);
+      scores(sg, sh, loads_in(tl, Next()));
+      loads_after(tl, Next(), 2 * KS);
+      __builtin_amdgcn_s_setprio(0);
+      softmax(sg, sh, pf, t);
+      __builtin_amdgcn_s_setprio(2);
+      pv(sg, pf, no_slot);
+    };
+    for (int t = t0; t < tend; t += 2) {
+      body(t, B0());
+      if (t + 1 < tend) body(t + 1, B1());
+    }
+  }
+  if (!SMALL && ntile > 0) {
     {
       using B0 = std::integral_constant<int, 0>;
       using B1 = std::integral_constant<int, 1>;
@@ -676,8 +717,14 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_kernel(FwdArgs a) {
   // products: 75,600 queries x 512 keys, fwd+bwd, 5.59 -> 5.29 ms with
   // the dQ kernel's, (2,20,3600,128) forward 331 -> 326 us).
   barrier_lds();
-  Stage& est = (wave & 3) == 0 ? st0 : ((wave & 3) == 1 ? st1 : ((wave & 3) == 2 ? st2 : st3));
-  bf16* ep = wave < 4 ? est.k : est.vt;
+  bf16* ep;
+  if constexpr (SMALL) {
+    Stage& est = wave & 1 ? st1 : st0;
+    ep = wave < 2 ? est.k : est.vt;
+  } else {
+    Stage& est = (wave & 3) == 0 ? st0 : ((wave & 3) == 1 ? st1 : ((wave & 3) == 2 ? st2 : st3));
+    ep = wave < 4 ? est.k : est.vt;
+  }
   static_assert(sizeof(st0.k) >= 32 * D * sizeof(bf16), "a wave's output rows fit a K stage");
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -758,6 +805,36 @@ __global__ void attn_empty_kernel(bf16* o, int64_t osb, int64_t osh, int64_t osl
   }
 }
 
+// Which workgroups a bf16 forward runs in.  Measured on one MI355X, 256-row
+// against 128-row (SMALL) workgroups:
+//   D 64, any shape: SMALL (three workgroups per CU): (2,20,16384) 2833 ->
+//     2617 us, (2,16,7176) 505 -> 467, 20,000 x 256 keys 51 -> 41, varlen
+//     (1,20,37800) 2645 -> 2380, window (1,20,21600) 1106 -> 963;
+//   D 128, many tiles per workgroup and several rounds of workgroups: 256
+//     rows ((2,20,16384) 4174 against 4630 us, (1,20,5265) 256 against 302,
+//     (2,40,2304) 220 against 236);
+//   D 128, few keys, where the prologue and output are a large part: SMALL
+//     (75,600 x 128 keys 521 -> 470 us, 20,000 x 256 74.7 -> 66.2, x 512
+//     within noise);
+//   D 128, at most one workgroup of 256 rows per CU: SMALL, which spreads
+//     over more CUs ((1,4,4096) 80.1 -> 75.5 us, (1,8,3000) 66.3 -> 62.6,
+//     (1,20,1024) 34.3 -> 32.0).
+constexpr int kSmallKeys = 512, kCus = 256;
+static bool use_small(const FwdArgs& a, int head_dim) {
+  return head_dim == 64 || a.Lk <= kSmallKeys || (int64_t)((a.Lq + 255) / 256) * a.B * a.Hq <= kCus;
+}
+
+template <int D, bool SMALL>
+static void launch_variant(const FwdArgs& a, dim3 grid, hipStream_t stream) {
+  const dim3 block(SMALL ? 256 : 512);
+  if (a.wlo != nullptr)
+    hipLaunchKernelGGL((attn_fwd_kernel<D, false, false, true, SMALL>), grid, block, 0, stream, a);
+  else if (a.cos_q != nullptr)
+    hipLaunchKernelGGL((attn_fwd_kernel<D, true, false, false, SMALL>), grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL((attn_fwd_kernel<D, false, false, false, SMALL>), grid, block, 0, stream, a);
+}
+
 template <int D>
 static hipError_t launch_fwd_d(const FwdArgs& a, hipStream_t stream) {
   const bool fp8 = a.k8 != nullptr;
@@ -767,18 +844,16 @@ static hipError_t launch_fwd_d(const FwdArgs& a, hipStream_t stream) {
     e = launch_quantize_rows(a.k, a.ksb, a.ksh, a.ksl, a.B, a.Hkv, a.Lk, D, a.k_scale, a.k8, a.kmax2, stream);
   }
   if (e != hipSuccess) return e;
-  const int nqt = (a.Lq + 255) / 256;
-  const dim3 grid(nqt * a.B * a.Hq);
-  const dim3 block(512);
   LaunchTimer timer(fp8 ? kKidFwdFp8 : kKidFwd, stream);
+  const bool small = !fp8 && use_small(a, D);
+  const int bm = small ? 128 : 256;
+  const dim3 grid((a.Lq + bm - 1) / bm * a.B * a.Hq);
   if (fp8)
-    hipLaunchKernelGGL((attn_fwd_kernel<D, false, true, false>), grid, block, 0, stream, a);
-  else if (a.wlo != nullptr)
-    hipLaunchKernelGGL((attn_fwd_kernel<D, false, false, true>), grid, block, 0, stream, a);
-  else if (a.cos_q != nullptr)
-    hipLaunchKernelGGL((attn_fwd_kernel<D, true, false, false>), grid, block, 0, stream, a);
-  else
-    hipLaunchKernelGGL((attn_fwd_kernel<D, false, false, false>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((attn_fwd_kernel<D, false, true, false, false>), grid, dim3(512), 0, stream, a);
+  else if (small)
+    launch_variant<D, true>(a, grid, stream);
+  else if constexpr (D != 64)  // never at D 64 (use_small)
+    launch_variant<D, false>(a, grid, stream);
   return hipGetLastError();
 }
 
