@@ -61,6 +61,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
          c_ptr],
     ),
     "avattn_fwd_workspace_size": (c_size, [c_i32, c_i32, c_i32, c_i32]),
+    "avattn_fwd_split_workspace_size": (c_size, [c_i32] * 7),
     "avattn_fwd_fp8": (
         ctypes.c_int,
         [c_ptr, c_ptr, c_ptr, c_i64p, c_i64p, c_i64p,

@@ -20,6 +20,96 @@
 
 namespace avattn {
 
+// Row state of a query from its reference max m (raw score units, or log2
+// units with fp8; `unit` converts it to natural log) and probability sum l:
+// l > 0; l == 0, no valid key (out 0 as SDPA returns, lse -inf); NaN, a NaN
+// (or +inf) score reached the row (out and lse NaN, as the softmax of such a
+// row gives).  inv scales the accumulated output.
+__device__ __forceinline__ void row_state(float m, float l, float unit, float& inv, float& lse) {
+  const float nan = __builtin_nanf("");
+  inv = l > 0.f ? 1.f / l : (l == 0.f ? 0.f : nan);
+  lse = l > 0.f ? fmaf(m, unit, logf(l)) : (l == 0.f ? kNegInf : nan);
+}
+
+// Writes one wave's 32 output rows row0 .. of (b, h) = bh: acc[dt][4*g + r] of
+// lane l is channel 32*dt + 8*g + 4*(l/32) + r of row l%32, times inv; lse
+// per lane row.
+// The output leaves through LDS (ep: 32*D elements nothing else
+// uses), so that each store instruction covers whole rows: in the C
+// layout a lane holds 4 consecutive channels, and a store would touch 32
+// rows for 16 bytes each (with few keys per row that cost more than the
+// products: 75,600 queries x 512 keys, fwd+bwd, 5.59 -> 5.29 ms with
+// the dQ kernel's, (2,20,3600,128) forward 331 -> 326 us).
+template <int D>
+__device__ __forceinline__ void write_rows(const FwdArgs& a, const f32x16 (&acc)[D / 32], float inv, float lse,
+                                           bf16* ep, int bh, int row0) {
+  constexpr int DT = D / 32;
+  const int lane = threadIdx.x & 63;
+  const int l32 = lane & 31, hh = lane >> 5;
+  const int b = bh / a.Hq, h = bh % a.Hq;
+  const bool qvalid = row0 + l32 < a.Lq;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      u32x2 w;
+      w[0] = pack_bf16x2(acc[dt][4 * g] * inv, acc[dt][4 * g + 1] * inv);
+      w[1] = pack_bf16x2(acc[dt][4 * g + 2] * inv, acc[dt][4 * g + 3] * inv);
+      *reinterpret_cast<u32x2*>(ep + TileLayout<D>::off(l32, dt * 32 + 8 * g) + 4 * hh) = w;
+    }
+  constexpr int kCpr = D / 8, kRpi = 64 / kCpr;  // chunks per row, rows per store
+  const int er = lane / kCpr, ec = 8 * (lane % kCpr);
+  bf16* op = a.o + b * a.osb + h * a.osh + ec;
+  if (a.o_acc == nullptr) {
+    if (qvalid && hh == 0) a.lse[(int64_t)bh * a.Lq + row0 + l32] = lse;
+#pragma unroll
+    for (int i = 0; i < 32 / kRpi; ++i) {
+      const int r = i * kRpi + er;
+      const u32x4 x = *reinterpret_cast<const u32x4*>(ep + TileLayout<D>::off(r, ec));
+      if (row0 + r < a.Lq) *reinterpret_cast<u32x4*>(op + (int64_t)(row0 + r) * a.osl) = x;
+    }
+  } else {
+    // Ring step: merge this chunk's bf16-rounded output and lse into the
+    // fp32 accumulator, exactly as lse_merge_kernel would merge them
+    // (torch/.../_context_parallel/_attention.py:182-183).
+    int mode = 1;
+    float w = 1.f;
+    float nl = lse;
+    const int64_t arow0 = (int64_t)bh * a.Lq + row0;
+    if (!a.acc_first && qvalid) nl = lse_merge_coeffs(a.lse_acc[arow0 + l32], lse, mode, w);
+#pragma unroll
+    for (int i = 0; i < 32 / kRpi; ++i) {
+      const int r = i * kRpi + er;
+      const int rmode = __shfl(mode, r);
+      const float rw = __shfl(w, r);
+      const u32x4 x = *reinterpret_cast<const u32x4*>(ep + TileLayout<D>::off(r, ec));
+      if (row0 + r < a.Lq) {
+        float* accp = a.o_acc + (arow0 + r) * D + ec;
+        f32x4 m[2] = {{bf16_lo(x[0]), bf16_hi(x[0]), bf16_lo(x[1]), bf16_hi(x[1])},
+                      {bf16_lo(x[2]), bf16_hi(x[2]), bf16_lo(x[3]), bf16_hi(x[3])}};
+        if (rmode != 1) {
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            const f32x4 prev = *reinterpret_cast<const f32x4*>(accp + 4 * p);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) m[p][e] = lse_merge_elem(prev[e], m[p][e], rmode, rw);
+          }
+        }
+        *reinterpret_cast<f32x4*>(accp) = m[0];
+        *reinterpret_cast<f32x4*>(accp + 4) = m[1];
+        if (a.acc_final) {
+          const u32x4 fo = {pack_bf16x2(m[0][0], m[0][1]), pack_bf16x2(m[0][2], m[0][3]),
+                            pack_bf16x2(m[1][0], m[1][1]), pack_bf16x2(m[1][2], m[1][3])};
+          *reinterpret_cast<u32x4*>(op + (int64_t)(row0 + r) * a.osl) = fo;
+        }
+      }
+    }
+    // Both lanes of the row read lse_acc above (one wave, program order)
+    // before this write.
+    if (qvalid && hh == 0) a.lse_acc[arow0 + l32] = nl;
+  }
+}
+
 // One workgroup = 256 query rows of one (batch, head), 8 waves x 32 rows, one
 // workgroup per CU; K/V tiles of 64 keys.  Waves 0-3 (group A) and 4-7
 // (group B) share the SIMDs pairwise and run the same per-tile work
@@ -90,8 +180,17 @@ __global__ __launch_bounds__(SMALL ? 256 : 512, SMALL ? 2 : 1) void attn_fwd_ker
   const int prow = perm23(l32);  // K row this lane supplies to S^T = K Q^T
 
   const int nqt = (a.Lq + BM - 1) / BM;
-  const int total = nqt * a.B * a.Hq;
-  const int bid = xcd_remap(blockIdx.x, total);
+  // Row blocks 0 .. nfull-1 take one workgroup each; the last a.nsplit (the
+  // grid's partial last round) a.nparts each, one per range of key tiles.
+  const int nfull = nqt * a.B * a.Hq - a.nsplit;
+  int bid, part = -1;
+  if ((int)blockIdx.x < nfull) {
+    bid = xcd_remap(blockIdx.x, nfull);
+  } else {
+    const int i = blockIdx.x - nfull;
+    bid = nfull + i / a.nparts;
+    part = i % a.nparts;
+  }
   const int qt = bid % nqt;
   const int bh = bid / nqt;
   const int b = bh / a.Hq, h = bh % a.Hq;
@@ -559,6 +658,11 @@ __global__ __launch_bounds__(SMALL ? 256 : 512, SMALL ? 2 : 1) void attn_fwd_ker
     for (int i = done; i < kStageOps; ++i) stage_op(t, nextc, i);
   };
 
+  if (part >= 0) {  // this part's share of the tiles (possibly none)
+    const int p0 = ntile * part / a.nparts, p1 = ntile * (part + 1) / a.nparts;
+    t0 += p0;
+    ntile = p1 - p0;
+  }
   const int tend = t0 + ntile;  // tiles t0 .. tend-1
   retire_prologue_loads();
   // ntile is the same for every wave of the workgroup (0: no key to visit).
@@ -702,20 +806,26 @@ __global__ __launch_bounds__(SMALL ? 256 : 512, SMALL ? 2 : 1) void attn_fwd_ker
   __builtin_amdgcn_s_setprio(0);
   wait_vmem();  // the last (re-staged) tile loads
 
-  // Three row states: l_tot > 0; l_tot == 0, no valid key (out 0 as SDPA
-  // returns, lse -inf); NaN, a NaN (or +inf) score reached the row (out and
-  // lse NaN, as the softmax of such a row gives).
   const float l_tot = halves_sum(l_run0 + l_run1);
-  const float nan = __builtin_nanf("");
-  const float inv = l_tot > 0.f ? 1.f / l_tot : (l_tot == 0.f ? 0.f : nan);
-  // m_run is in raw score units (bf16 path) or log2 units (fp8).
-  const float lse = l_tot > 0.f ? fmaf(m_run, FP8 ? kLn2 : sc, logf(l_tot)) : (l_tot == 0.f ? kNegInf : nan);
-  // The output leaves through LDS (this wave's 32 rows in a stage no wave reads
-  // any more), so that each store instruction covers whole rows: in the C
-  // layout a lane holds 4 consecutive channels, and a store would touch 32
-  // rows for 16 bytes each (with few keys per row that cost more than the
-  // products: 75,600 queries x 512 keys, fwd+bwd, 5.59 -> 5.29 ms with
-  // the dQ kernel's, (2,20,3600,128) forward 331 -> 326 us).
+  if (part >= 0) {
+    // One part of split rows: the raw accumulators, max and sum, in the lane
+    // order fwd_combine_kernel reads them back in.
+    float* slot = a.part + ((int64_t)(bid - nfull) * a.nparts + part) * fwd_slot_floats(BM, D) +
+                  (int64_t)wave * fwd_slot_floats(32, D);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4*>(slot + ((dt * 4 + g) * 64 + lane) * 4) =
+            f32x4{acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]};
+    if (hh == 0) {
+      slot[32 * D + l32] = m_run;
+      slot[32 * D + 32 + l32] = l_tot;
+    }
+    return;
+  }
+  float inv, lse;
+  row_state(m_run, l_tot, FP8 ? kLn2 : sc, inv, lse);
   barrier_lds();
   bf16* ep;
   if constexpr (SMALL) {
@@ -726,67 +836,50 @@ __global__ __launch_bounds__(SMALL ? 256 : 512, SMALL ? 2 : 1) void attn_fwd_ker
     ep = wave < 4 ? est.k : est.vt;
   }
   static_assert(sizeof(st0.k) >= 32 * D * sizeof(bf16), "a wave's output rows fit a K stage");
+  write_rows<D>(a, acc, inv, lse, ep, bh, qt * BM + wave * 32);
+}
+
+// The split row blocks (FwdArgs::nsplit): one wave per 32 rows adds the
+// parts in order, each scaled from its own reference max to the largest, and
+// writes the rows as the forward's own epilogue does.  BM: rows per block.
+template <int D, int BM>
+__global__ __launch_bounds__(256) void fwd_combine_kernel(FwdArgs a, float c, float unit) {
+  constexpr int DT = D / 32;
+  __shared__ __attribute__((aligned(16))) bf16 ep[4][32 * D];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l32 = lane & 31;
+  const int u = blockIdx.x * 4 + wave;  // 32-row group of the split blocks
+  const int s = u / (BM / 32), w = u % (BM / 32);
+  const int nqt = (a.Lq + BM - 1) / BM;
+  const int bid = nqt * a.B * a.Hq - a.nsplit + s;
+  const int row0 = bid % nqt * BM + w * 32;
+  const float* slot = a.part + (int64_t)s * a.nparts * fwd_slot_floats(BM, D) + (int64_t)w * fwd_slot_floats(32, D);
+  float m = kNegInf;
+  for (int p = 0; p < a.nparts; ++p) m = fmaxf(m, slot[p * fwd_slot_floats(BM, D) + 32 * D + l32]);
+  float l = 0.f;
+  f32x16 acc[DT];
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
+  for (int i = 0; i < DT; ++i) acc[i] = zero16();
+  for (int p = 0; p < a.nparts; ++p) {
+    const float* sp = slot + p * fwd_slot_floats(BM, D);
+    const float mp = sp[32 * D + l32];
+    // a part without an attended key (mp -inf) weighs nothing, unless a NaN
+    // reached its sum or output
+    const float wt = mp == kNegInf ? 0.f : __builtin_amdgcn_exp2f((mp - m) * c);
+    l = fmaf(sp[32 * D + 32 + l32], wt, l);
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      u32x2 w;
-      w[0] = pack_bf16x2(acc[dt][4 * g] * inv, acc[dt][4 * g + 1] * inv);
-      w[1] = pack_bf16x2(acc[dt][4 * g + 2] * inv, acc[dt][4 * g + 3] * inv);
-      *reinterpret_cast<u32x2*>(ep + TileLayout<D>::off(l32, dt * 32 + 8 * g) + 4 * hh) = w;
-    }
-  constexpr int kCpr = D / 8, kRpi = 64 / kCpr;  // chunks per row, rows per store
-  const int er = lane / kCpr, ec = 8 * (lane % kCpr);
-  const int row0 = qt * BM + wave * 32;
-  bf16* op = a.o + b * a.osb + h * a.osh + ec;
-  if (a.o_acc == nullptr) {
-    if (qvalid && hh == 0) a.lse[(int64_t)bh * a.Lq + qrow] = lse;
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int i = 0; i < 32 / kRpi; ++i) {
-      const int r = i * kRpi + er;
-      const u32x4 x = *reinterpret_cast<const u32x4*>(ep + TileLayout<D>::off(r, ec));
-      if (row0 + r < a.Lq) *reinterpret_cast<u32x4*>(op + (int64_t)(row0 + r) * a.osl) = x;
-    }
-  } else {
-    // Ring step: merge this chunk's bf16-rounded output and lse into the
-    // fp32 accumulator, exactly as lse_merge_kernel would merge them
-    // (torch/.../_context_parallel/_attention.py:182-183).
-    int mode = 1;
-    float w = 1.f;
-    float nl = lse;
-    const int64_t arow0 = (int64_t)bh * a.Lq + row0;
-    if (!a.acc_first && qvalid) nl = lse_merge_coeffs(a.lse_acc[arow0 + l32], lse, mode, w);
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(sp + ((dt * 4 + g) * 64 + lane) * 4);
 #pragma unroll
-    for (int i = 0; i < 32 / kRpi; ++i) {
-      const int r = i * kRpi + er;
-      const int rmode = __shfl(mode, r);
-      const float rw = __shfl(w, r);
-      const u32x4 x = *reinterpret_cast<const u32x4*>(ep + TileLayout<D>::off(r, ec));
-      if (row0 + r < a.Lq) {
-        float* accp = a.o_acc + (arow0 + r) * D + ec;
-        f32x4 m[2] = {{bf16_lo(x[0]), bf16_hi(x[0]), bf16_lo(x[1]), bf16_hi(x[1])},
-                      {bf16_lo(x[2]), bf16_hi(x[2]), bf16_lo(x[3]), bf16_hi(x[3])}};
-        if (rmode != 1) {
-#pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            const f32x4 prev = *reinterpret_cast<const f32x4*>(accp + 4 * p);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) m[p][e] = lse_merge_elem(prev[e], m[p][e], rmode, rw);
-          }
-        }
-        *reinterpret_cast<f32x4*>(accp) = m[0];
-        *reinterpret_cast<f32x4*>(accp + 4) = m[1];
-        if (a.acc_final) {
-          const u32x4 fo = {pack_bf16x2(m[0][0], m[0][1]), pack_bf16x2(m[0][2], m[0][3]),
-                            pack_bf16x2(m[1][0], m[1][1]), pack_bf16x2(m[1][2], m[1][3])};
-          *reinterpret_cast<u32x4*>(op + (int64_t)(row0 + r) * a.osl) = fo;
-        }
+        for (int r = 0; r < 4; ++r) acc[dt][4 * g + r] = fmaf(x[r], wt, acc[dt][4 * g + r]);
       }
-    }
-    // Both lanes of the row read lse_acc above (one wave, program order)
-    // before this write.
-    if (qvalid && hh == 0) a.lse_acc[arow0 + l32] = nl;
   }
+  float inv, lse;
+  row_state(m, l, unit, inv, lse);
+  write_rows<D>(a, acc, inv, lse, ep[wave], bid / nqt, row0);
 }
 
 // Writes zeros to out and -inf to lse: attention over an empty key set
@@ -820,8 +913,49 @@ __global__ void attn_empty_kernel(bf16* o, int64_t osb, int64_t osh, int64_t osl
 //     over more CUs ((1,4,4096) 80.1 -> 75.5 us, (1,8,3000) 66.3 -> 62.6,
 //     (1,20,1024) 34.3 -> 32.0).
 constexpr int kSmallKeys = 512, kCus = 256;
-static bool use_small(const FwdArgs& a, int head_dim) {
-  return head_dim == 64 || a.Lk <= kSmallKeys || (int64_t)((a.Lq + 255) / 256) * a.B * a.Hq <= kCus;
+static bool use_small(int B, int Hq, int Lq, int Lk, int head_dim) {
+  return head_dim == 64 || Lk <= kSmallKeys || (int64_t)((Lq + 255) / 256) * B * Hq <= kCus;
+}
+
+// Split of the last round's row blocks over ranges of key tiles: the number
+// of parts (2..8, at least 8 tiles each) with the smallest estimated time, if
+// it saves 4 us or more.  Times per tile and round and per workgroup as
+// measured on an MI355X; (1,4,4096,128) 78.7 -> 61.1 us, D 64 56.7 -> 41.0,
+// (1,16,4725,128) x 18,900 keys 844 -> 666, (1,8,18900,128) 1330 -> 1190.
+FwdSplit fwd_split_plan(int B, int Hq, int Lq, int Lk, int D, bool fp8, bool windows) {
+  FwdSplit best{0, 0, 0};
+  if (windows) return best;  // the tiles of a row block are known on the device only
+  const bool small = !fp8 && use_small(B, Hq, Lq, Lk, D);
+  const int bm = small ? 128 : 256;
+  const int per_cu = small ? (D == 64 ? 3 : 2) : 1;
+  const int slots = kCus * per_cu;
+  const int ntile = (Lk + 63) / 64;
+  const int r = (int)((int64_t)((Lq + bm - 1) / bm) * B * Hq % slots);
+  const float tile_us = fp8 ? 1.25f : (D == 64 ? 1.55f : 1.7f), fixed_us = 8.f;
+  // Rounds n workgroups take.  A partial round is shorter than a full one:
+  // one workgroup on a CU by itself takes less than per_cu sharing it, and
+  // the chip, power-limited when full, clocks higher with CUs idle (measured:
+  // splitting 80 workgroups of 295 tiles left after two rounds saved 140 us
+  // of 1330, where full-length rounds would have made it 335).
+  auto rounds = [&](int n) {
+    const int rem = n % slots;
+    if (rem == 0) return (float)(n / slots);
+    const int k = (rem + kCus - 1) / kCus;
+    const float idle = 1.f - (float)rem / (k * kCus);
+    return n / slots + (k + 0.2f * (per_cu - k)) / per_cu * (1.f - (small ? 0.25f : 0.38f) * idle);
+  };
+  // The parts cost their partial sums, written and read at 4 TB/s, and the
+  // combining launch.
+  const float slot_bytes = 4.f * fwd_slot_floats(bm, D);
+  float cost = rounds(r) * (ntile * tile_us + fixed_us) - 4.f;
+  for (int p = 2; p <= 8 && ntile / p >= 8; ++p) {
+    const float c = rounds(r * p) * (ntile * tile_us / p + fixed_us) + 5.f + r * p * slot_bytes * 0.5e-6f;
+    if (c < cost) {
+      cost = c;
+      best = FwdSplit{r, p, (size_t)r * p * fwd_slot_floats(bm, D) * sizeof(float)};
+    }
+  }
+  return best;
 }
 
 template <int D, bool SMALL>
@@ -836,7 +970,8 @@ static void launch_variant(const FwdArgs& a, dim3 grid, hipStream_t stream) {
 }
 
 template <int D>
-static hipError_t launch_fwd_d(const FwdArgs& a, hipStream_t stream) {
+static hipError_t launch_fwd_d(const FwdArgs& args, hipStream_t stream) {
+  FwdArgs a = args;
   const bool fp8 = a.k8 != nullptr;
   hipError_t e = launch_prep_fwd(a, D, stream);
   if (e == hipSuccess && fp8) {
@@ -844,16 +979,32 @@ static hipError_t launch_fwd_d(const FwdArgs& a, hipStream_t stream) {
     e = launch_quantize_rows(a.k, a.ksb, a.ksh, a.ksl, a.B, a.Hkv, a.Lk, D, a.k_scale, a.k8, a.kmax2, stream);
   }
   if (e != hipSuccess) return e;
-  LaunchTimer timer(fp8 ? kKidFwdFp8 : kKidFwd, stream);
-  const bool small = !fp8 && use_small(a, D);
+  const bool small = !fp8 && use_small(a.B, a.Hq, a.Lq, a.Lk, D);
   const int bm = small ? 128 : 256;
-  const dim3 grid((a.Lq + bm - 1) / bm * a.B * a.Hq);
-  if (fp8)
-    hipLaunchKernelGGL((attn_fwd_kernel<D, false, true, false, false>), grid, dim3(512), 0, stream, a);
-  else if (small)
-    launch_variant<D, true>(a, grid, stream);
-  else if constexpr (D != 64)  // never at D 64 (use_small)
-    launch_variant<D, false>(a, grid, stream);
+  const int64_t blocks = (int64_t)((a.Lq + bm - 1) / bm) * a.B * a.Hq;
+  const FwdSplit sp = fwd_split_plan(a.B, a.Hq, a.Lq, a.Lk, D, fp8, a.wlo != nullptr);
+  if (a.part != nullptr) {
+    a.nsplit = sp.nsplit;
+    a.nparts = sp.nparts;
+  }
+  const dim3 grid((unsigned)(blocks - a.nsplit + (int64_t)a.nsplit * a.nparts));
+  {
+    LaunchTimer timer(fp8 ? kKidFwdFp8 : kKidFwd, stream);
+    if (fp8)
+      hipLaunchKernelGGL((attn_fwd_kernel<D, false, true, false, false>), grid, dim3(512), 0, stream, a);
+    else if (small)
+      launch_variant<D, true>(a, grid, stream);
+    else if constexpr (D != 64)  // never at D 64 (use_small)
+      launch_variant<D, false>(a, grid, stream);
+  }
+  if (a.nsplit > 0) {
+    const float c = fp8 ? 1.f : a.scale_log2, unit = fp8 ? kLn2 : a.scale;
+    LaunchTimer timer(kKidMerge, stream);
+    if (small)
+      hipLaunchKernelGGL((fwd_combine_kernel<D, 128>), dim3(a.nsplit), dim3(256), 0, stream, a, c, unit);
+    else
+      hipLaunchKernelGGL((fwd_combine_kernel<D, 256>), dim3(2 * a.nsplit), dim3(256), 0, stream, a, c, unit);
+  }
   return hipGetLastError();
 }
 

@@ -283,6 +283,10 @@ int fwd_impl(const void* q, const void* k, const void* v, const int64_t* q_strid
   a.wlo = window_lo;
   a.whi = window_hi;
   a.wsb = window_batch_stride;
+  // A workspace of avattn_fwd_split_workspace_size bytes holds the parts of a
+  // split last round; a smaller one runs the unsplit grid.
+  const size_t split = fwd_split_plan(batch, heads_q, len_q, len_k, head_dim, fp8, window_lo != nullptr).bytes;
+  if (split > 0 && workspace_bytes >= wl.total + split) a.part = reinterpret_cast<float*>(ws + wl.total);
   if (ring) {
     a.cos_k = ring->cos_k;
     a.sin_k = ring->sin_k;
@@ -357,6 +361,14 @@ int avattn_fp8_absmax_scales(const void* x, const int64_t* x_strides, int32_t ba
 size_t avattn_fwd_workspace_size(int32_t batch, int32_t heads_kv, int32_t len_k, int32_t head_dim) {
   if (batch <= 0 || heads_kv <= 0 || len_k <= 0 || head_dim <= 0) return 0;
   return fwd_workspace(batch, heads_kv, len_k, head_dim).total;
+}
+
+size_t avattn_fwd_split_workspace_size(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t len_q, int32_t len_k,
+                                       int32_t head_dim, int32_t fp8) {
+  if (check_dims(batch, heads_q, heads_kv, len_q, len_k, head_dim) != AVATTN_OK) return 0;
+  if ((int64_t)batch * heads_q * len_q == 0 || len_k == 0) return 0;
+  return fwd_workspace(batch, heads_kv, len_k, head_dim, fp8 != 0).total +
+         fwd_split_plan(batch, heads_q, len_q, len_k, head_dim, fp8 != 0, false).bytes;
 }
 
 size_t avattn_bwd_workspace_size(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t len_q, int32_t len_k,
@@ -877,5 +889,5 @@ extern "C" int avattn_fwd_noalloc(const void* q, const void* k, const void* v, c
   }
   return fwd_impl(q, k, v, q_strides, k_strides, v_strides, batch, heads_q, heads_kv, len_q, len_k, head_dim,
                   key_mask, key_mask_batch_stride, rope_cos_q, rope_sin_q, rope_batch_stride, false, nullptr,
-                  nullptr, scale, out, out_strides, lse, ws, ws ? AVATTN_FWD_NOALLOC_SCRATCH : 0, stream);
+                  nullptr, scale, out, out_strides, lse, ws, ws ? need : 0, stream);
 }

@@ -72,7 +72,25 @@ struct FwdArgs {
   float* lse_acc;
   bool acc_first;
   bool acc_final;
+  // Split of the grid's partial last round (null part: none; nsplit and
+  // nparts are set by launch_fwd from fwd_split_plan): the last nsplit row
+  // blocks each go to nparts workgroups, one per range of key tiles, which
+  // store their accumulators, max and sum in slot (block - first split
+  // block) * nparts + part of fwd_slot_floats floats; a combining kernel
+  // writes the rows.
+  float* part;
+  int nsplit, nparts;
 };
+
+// Floats of one part of `rows` rows: the accumulators, then per 32 rows their
+// maxima and sums.
+constexpr int fwd_slot_floats(int rows, int D) { return rows * (D + 2); }
+// The forward's split for a shape (nsplit 0: none) and the bytes of its slots.
+struct FwdSplit {
+  int nsplit, nparts;
+  size_t bytes;
+};
+FwdSplit fwd_split_plan(int B, int Hq, int Lq, int Lk, int head_dim, bool fp8, bool windows);
 
 struct BwdArgs {
   const bf16* dout;

@@ -191,7 +191,7 @@ def _fwd_impl(q, k, v, key_mask, rope_cos, rope_sin, scale):
     out = _kernel_ready(out)
     lse = torch.empty((B, Hq, Lq), device=q.device, dtype=torch.float32)
     lib = _lib.load()
-    ws = _workspace(lib.avattn_fwd_workspace_size(B, Hkv, Lk, D), q.device)
+    ws = _workspace(lib.avattn_fwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D, 0), q.device)
     st = lib.avattn_fwd(
         _ptr(q), _ptr(k), _ptr(v), _strides3(q), _strides3(k), _strides3(v),
         B, Hq, Hkv, Lq, Lk, D,
@@ -453,7 +453,7 @@ def _fwd_fp8_impl(q, k, v, key_mask, q_scale, k_scale, scale):
     out = _kernel_ready(torch.empty_like(q, memory_format=torch.preserve_format))
     lse = torch.empty((B, Hq, Lq), device=q.device, dtype=torch.float32)
     lib = _lib.load()
-    ws = _workspace(lib.avattn_fwd_fp8_workspace_size(B, Hkv, Lk, D), q.device)
+    ws = _workspace(lib.avattn_fwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D, 1), q.device)
     st = lib.avattn_fwd_fp8(
         _ptr(q), _ptr(k), _ptr(v), _strides3(q), _strides3(k), _strides3(v),
         B, Hq, Hkv, Lq, Lk, D,
@@ -785,7 +785,7 @@ def _ring_fwd_step_impl(q, k, v, key_mask, cos_q, sin_q, cos_k, sin_k, scale, ou
     ck, sk, rksb = _ring_tables(name, cos_k, sin_k, B, Lk, D)
     flags = (_lib.RING_FIRST if first else 0) | (_lib.RING_LAST if last else 0)
     lib = _lib.load()
-    ws = _workspace(lib.avattn_fwd_workspace_size(B, Hkv, Lk, D), q.device)
+    ws = _workspace(lib.avattn_fwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D, 0), q.device)
     st = lib.avattn_ring_fwd_step(
         _ptr(q), _ptr(k), _ptr(v), _strides3(q), _strides3(k), _strides3(v),
         B, Hq, Hkv, Lq, Lk, D,

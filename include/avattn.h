@@ -152,6 +152,18 @@ int avattn_fwd_noalloc(const void* q, const void* k, const void* v,
 size_t avattn_fwd_workspace_size(int32_t batch, int32_t heads_kv, int32_t len_k, int32_t head_dim);
 
 /*
+ * Workspace with which avattn_fwd, avattn_ring_fwd_step (fp8 0) and
+ * avattn_fwd_fp8 (fp8 nonzero) also split the partial last round of their
+ * grid over ranges of keys where that is faster: the base size plus the
+ * parts' partial sums (0 for a problem the forward would refuse or that is
+ * empty).  With a smaller workspace of at least the base size they run
+ * unsplit; the split rows differ in the last rounding only.  Reproducible
+ * bit for bit for a given workspace size either way.
+ */
+size_t avattn_fwd_split_workspace_size(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t len_q, int32_t len_k,
+                                       int32_t head_dim, int32_t fp8);
+
+/*
  * Workspace bytes avattn_bwd needs for these sizes: two floats per query row
  * (softmax statistics), row-major copies of q and dout,
  * row-major copies of k and v and a head_dim-major copy of k (sequences

@@ -1,0 +1,64 @@
+"""The forward with its last round split over ranges of keys against the
+unsplit one: the same result up to the rounding of the merge, and the row
+states (no attended key, NaN) merged exactly."""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _call(lib, q, k, v, mask, nbytes):
+    from avgen_amd import ops
+
+    B, H, Lq, D = q.shape
+    out, lse = torch.empty_like(q), torch.empty((B, H, Lq), device="cuda")
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    st = lib.avattn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), ops._strides3(q), ops._strides3(k), ops._strides3(v),
+                        B, H, k.shape[1], Lq, k.shape[2], D, None if mask is None else mask.data_ptr(),
+                        0 if mask is None else mask.stride(0), None, None, 0, 1.0 / math.sqrt(D), out.data_ptr(),
+                        ops._strides3(out), lse.data_ptr(), ws.data_ptr(), ws.numel(),
+                        torch.cuda.current_stream().cuda_stream)
+    assert st == 0
+    return out, lse
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("B,H,Lq,Lk,D", [
+    (1, 4, 1024, 4096, 64),     # every block split
+    (2, 2, 1000, 4097, 128),    # ragged rows and keys
+    (1, 16, 4725, 5000, 128),   # full rounds of 256-row blocks, then a split one
+    (1, 31, 3201, 2049, 64),
+])
+def test_split_equals_unsplit(B, H, Lq, Lk, D, masked):
+    from avgen_amd import _lib
+
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(Lq)
+    q, k, v = (torch.randn(B, H, n, D, device="cuda", generator=g).to(torch.bfloat16) for n in (Lq, Lk, Lk))
+    k[:, :, -1] *= 4  # a late key raises the reference max of the last part only
+    mask = None
+    if masked:
+        mask = torch.rand(B, Lk, device="cuda", generator=g) > 0.3
+        mask[:, : Lk // 2] = False  # parts without an attended key
+        if B > 1:
+            mask[1] = False
+        mask = mask.view(torch.uint8)
+    if not masked:
+        q[0, 0, 5, 3] = float("nan")
+    base = lib.avattn_fwd_workspace_size(B, H, Lk, D)
+    split = lib.avattn_fwd_split_workspace_size(B, H, H, Lq, Lk, D, 0)
+    assert split > base
+    (o1, l1), (o2, l2) = _call(lib, q, k, v, mask, split), _call(lib, q, k, v, mask, base)
+    assert torch.equal(o1.isnan(), o2.isnan()) and torch.equal(l1.isnan(), l2.isnan())
+    assert torch.equal(l1 == float("-inf"), l2 == float("-inf"))
+    # one bf16 rounding of P (2^-9 of each term) and of the output apart
+    d = (o1.float() - o2.float()).nan_to_num(0.0).abs()
+    assert (d <= 2.0**-7 * o2.float().nan_to_num(0.0).abs() + 2.0**-8).all()
+    f = torch.isfinite(l2)
+    assert (l1[f] - l2[f]).abs().max() <= 1e-5 * l2[f].abs().max() if f.any() else True
+    if masked and B > 1:
+        assert (o1[1] == 0).all()
+    assert torch.equal(_call(lib, q, k, v, mask, split)[0].view(torch.int16), o1.view(torch.int16))
