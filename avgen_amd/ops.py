@@ -76,11 +76,73 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+_Strides3 = ctypes.c_int64 * 3
 
 
 def _strides3(t: torch.Tensor) -> ctypes.Array:
-    return _lib.i64_array(t.stride()[:3])
+    return _Strides3(*t.stride()[:3])
+
+
+# Plain eager calls go straight to an autograd function (or, without grad, to
+# the implementation) instead of through the dispatcher's Python op layers,
+# which cost 20-40 us a call, and again in the backward: a (1,1024,4x64) block
+# with q/k norm and rotation, host-bound at 590 us forward and backward for
+# 130 us of kernels, takes 440 (a two-chunk ring of 1,024 tokens 534 -> 337,
+# 1,024 x 128 keys 305 -> 216).  Whatever the op layer exists for keeps it: a traced or compiled
+# call, a dispatch or function mode (selective checkpointing, fake tensors),
+# vmap and the other function transforms, forward-mode tangents, tensor
+# subclasses and wrappers, any device but the GPU, and calls under a profiler
+# (whose traces name the ops).
+_plain_keys: frozenset[int] = frozenset()
+
+
+def _plain_eager(*tensors: Optional[torch.Tensor]) -> bool:
+    global _plain_keys
+    if torch.compiler.is_compiling():
+        return False
+    if (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
+            or torch.autograd._profiler_enabled()):
+        return False
+    for t in tensors:
+        if t is None:
+            continue
+        if (type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or not t.is_cuda:
+            return False
+        if torch._C._dispatch_keys(t).raw_repr() not in _plain_keys:
+            if _plain_keys:
+                return False
+            # The key sets of an ordinary tensor, made in and out of inference
+            # mode (process constants, not an input's).
+            keys = []
+            for inference in (False, True):
+                with torch.inference_mode(inference):
+                    keys.append(torch._C._dispatch_keys(torch.empty(0, device=t.device)).raw_repr())
+            _plain_keys = frozenset(keys)
+            if torch._C._dispatch_keys(t).raw_repr() not in _plain_keys:
+                return False
+    return True
+
+
+def _direct(function, op, impl, args, tensors):
+    """The op on ``args`` (``tensors``: its tensor arguments): directly when
+    :func:`_plain_eager`, through the dispatcher otherwise."""
+    if not _plain_eager(*tensors):
+        return op(*args)
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors):
+        return function.apply(*args)
+    return impl(*args)
+
+
+def _grad_direct(*tensors) -> bool:
+    """Whether a backward formula may call an implementation instead of its
+    op: plain eager and not itself differentiated (create_graph)."""
+    return not torch.is_grad_enabled() and _plain_eager(*tensors)
 
 
 def _workspace(nbytes: int, device: torch.device) -> torch.Tensor:
@@ -126,8 +188,10 @@ def _check_qkv(name: str, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, all
 
 def _kernel_ready(t: torch.Tensor) -> torch.Tensor:
     """Make the last dim contiguous and row starts 16-byte aligned."""
-    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0
-    ok = ok and all(s % 8 == 0 or n == 1 for s, n in zip(t.stride()[:3], t.shape[:3]))
+    s0, s1, s2, s3 = t.stride()
+    ok = s3 == 1 and t.data_ptr() % 16 == 0
+    if ok and (s0 | s1 | s2) % 8:
+        ok = all(s % 8 == 0 or n == 1 for s, n in zip((s0, s1, s2), t.shape[:3]))
     return t if ok else t.contiguous()
 
 
@@ -1065,7 +1129,7 @@ def _qk_norm_rope_bwd_impl(dy, x, weight, eps, cos, sin):
 
 
 @torch.library.custom_op("avgen_amd::flash_fwd", mutates_args=())
-def flash_fwd(
+def _flash_fwd_op(
     q: torch.Tensor,
     k: torch.Tensor,
     v: torch.Tensor,
@@ -1078,13 +1142,27 @@ def flash_fwd(
     return _fwd_impl(q, k, v, key_mask, rope_cos, rope_sin, scale)
 
 
-@flash_fwd.register_fake
+@_flash_fwd_op.register_fake
 def _(q, k, v, key_mask, rope_cos, rope_sin, scale):
     return torch.empty_like(q), q.new_empty((q.shape[0], q.shape[1], q.shape[2]), dtype=torch.float32)
 
 
+def flash_fwd(
+    q: torch.Tensor,
+    k: torch.Tensor,
+    v: torch.Tensor,
+    key_mask: Optional[torch.Tensor],
+    rope_cos: Optional[torch.Tensor],
+    rope_sin: Optional[torch.Tensor],
+    scale: float,
+) -> tuple[torch.Tensor, torch.Tensor]:
+    """Attention forward over one KV chunk: ``(out, lse)``; see module docstring."""
+    return _direct(_FlashFwd, _flash_fwd_op, _fwd_impl, (q, k, v, key_mask, rope_cos, rope_sin, scale),
+                   (q, k, v, key_mask, rope_cos, rope_sin))
+
+
 @torch.library.custom_op("avgen_amd::flash_bwd", mutates_args=())
-def flash_bwd(
+def _flash_bwd_op(
     dout: torch.Tensor,
     q: torch.Tensor,
     k: torch.Tensor,
@@ -1098,20 +1176,41 @@ def flash_bwd(
     return _bwd_impl(dout, q, k, v, out, lse, key_mask, scale)
 
 
-@flash_bwd.register_fake
+@_flash_bwd_op.register_fake
 def _(dout, q, k, v, out, lse, key_mask, scale):
     return torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
 
 
+def flash_bwd(
+    dout: torch.Tensor,
+    q: torch.Tensor,
+    k: torch.Tensor,
+    v: torch.Tensor,
+    out: torch.Tensor,
+    lse: torch.Tensor,
+    key_mask: Optional[torch.Tensor],
+    scale: float,
+) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """Attention backward over one KV chunk given the (possibly merged) out/lse."""
+    if _grad_direct(dout, q, k, v, out, lse, key_mask):
+        return _bwd_impl(dout, q, k, v, out, lse, key_mask, scale)
+    return _flash_bwd_op(dout, q, k, v, out, lse, key_mask, scale)
+
+
 @torch.library.custom_op("avgen_amd::rope_apply", mutates_args=())
-def rope_apply(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, inverse: bool) -> torch.Tensor:
+def _rope_apply_op(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, inverse: bool) -> torch.Tensor:
     """Interleaved-pair rotation (or its transpose) of ``x``."""
     return _rope_apply_impl(x, cos, sin, inverse)
 
 
-@rope_apply.register_fake
+@_rope_apply_op.register_fake
 def _(x, cos, sin, inverse):
     return x.new_empty(x.shape)
+
+
+def rope_apply(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, inverse: bool) -> torch.Tensor:
+    """Interleaved-pair rotation (or its transpose) of ``x``."""
+    return _direct(_RopeApply, _rope_apply_op, _rope_apply_impl, (x, cos, sin, inverse), (x, cos, sin))
 
 
 @torch.library.custom_op("avgen_amd::flash_fwd_fp8", mutates_args=())
@@ -1134,7 +1233,7 @@ def _(q, k, v, key_mask, q_scale, k_scale, scale):
 
 
 @torch.library.custom_op("avgen_amd::flash_fwd_windowed", mutates_args=())
-def flash_fwd_windowed(
+def _flash_fwd_windowed_op(
     q: torch.Tensor,
     k: torch.Tensor,
     v: torch.Tensor,
@@ -1150,13 +1249,35 @@ def flash_fwd_windowed(
     return _fwd_windowed_impl(q, k, v, window_lo, window_hi, key_mask, scale)
 
 
-@flash_fwd_windowed.register_fake
+@_flash_fwd_windowed_op.register_fake
 def _(q, k, v, window_lo, window_hi, key_mask, scale, monotone=False):
     return torch.empty_like(q), q.new_empty((q.shape[0], q.shape[1], q.shape[2]), dtype=torch.float32)
 
 
+def flash_fwd_windowed(
+    q: torch.Tensor,
+    k: torch.Tensor,
+    v: torch.Tensor,
+    window_lo: torch.Tensor,
+    window_hi: torch.Tensor,
+    key_mask: Optional[torch.Tensor],
+    scale: float,
+    monotone: bool = False,
+) -> tuple[torch.Tensor, torch.Tensor]:
+    """Forward where query row i attends keys [window_lo[i], window_hi[i]) only.
+    ``monotone``: the caller guarantees both bounds non-decreasing in the row
+    (its backward then skips the check and its host synchronisation)."""
+    return _direct(_FlashFwdWindowed, _flash_fwd_windowed_op, _fwd_windowed_fwd,
+                   (q, k, v, window_lo, window_hi, key_mask, scale, monotone),
+                   (q, k, v, window_lo, window_hi, key_mask))
+
+
+def _fwd_windowed_fwd(q, k, v, window_lo, window_hi, key_mask, scale, monotone):
+    return _fwd_windowed_impl(q, k, v, window_lo, window_hi, key_mask, scale)
+
+
 @torch.library.custom_op("avgen_amd::flash_bwd_windowed", mutates_args=())
-def flash_bwd_windowed(
+def _flash_bwd_windowed_op(
     dout: torch.Tensor,
     q: torch.Tensor,
     k: torch.Tensor,
@@ -1175,9 +1296,30 @@ def flash_bwd_windowed(
                               check_monotone=not monotone)
 
 
-@flash_bwd_windowed.register_fake
+@_flash_bwd_windowed_op.register_fake
 def _(dout, q, k, v, out, lse, window_lo, window_hi, key_mask, scale, monotone=False):
     return torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+
+
+def flash_bwd_windowed(
+    dout: torch.Tensor,
+    q: torch.Tensor,
+    k: torch.Tensor,
+    v: torch.Tensor,
+    out: torch.Tensor,
+    lse: torch.Tensor,
+    window_lo: torch.Tensor,
+    window_hi: torch.Tensor,
+    key_mask: Optional[torch.Tensor],
+    scale: float,
+    monotone: bool = False,
+) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """Backward of ``flash_fwd_windowed`` (windows non-decreasing in the row;
+    checked unless ``monotone``)."""
+    if _grad_direct(dout, q, k, v, out, lse, window_lo, window_hi, key_mask):
+        return _bwd_windowed_impl(dout, q, k, v, out, lse, window_lo, window_hi, key_mask, scale,
+                                  check_monotone=not monotone)
+    return _flash_bwd_windowed_op(dout, q, k, v, out, lse, window_lo, window_hi, key_mask, scale, monotone)
 
 
 def _fwd_windowed_setup(ctx, inputs, output):
@@ -1201,8 +1343,21 @@ torch.library.register_autograd(
 )
 
 
+class _FlashFwdWindowed(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, *args):
+        result = _fwd_windowed_fwd(*args)
+        ctx.set_materialize_grads(False)
+        _fwd_windowed_setup(ctx, args, result)
+        return result
+
+    @staticmethod
+    def backward(ctx, dout, _dlse):
+        return (None,) * 8 if dout is None else _fwd_windowed_backward(ctx, dout, None)
+
+
 @torch.library.custom_op("avgen_amd::qk_norm_rope", mutates_args=())
-def qk_norm_rope(
+def _qk_norm_rope_op(
     x: torch.Tensor, weight: Optional[torch.Tensor], eps: float, cos: Optional[torch.Tensor],
     sin: Optional[torch.Tensor],
 ) -> torch.Tensor:
@@ -1211,22 +1366,46 @@ def qk_norm_rope(
     return _qk_norm_rope_impl(x, weight, eps, cos, sin)
 
 
-@qk_norm_rope.register_fake
+@_qk_norm_rope_op.register_fake
 def _(x, weight, eps, cos, sin):
     return torch.empty_like(x)
 
 
+def qk_norm_rope(
+    x: torch.Tensor, weight: Optional[torch.Tensor], eps: float, cos: Optional[torch.Tensor],
+    sin: Optional[torch.Tensor],
+) -> torch.Tensor:
+    """Per-head RMSNorm (gain ``weight`` cast to the input's dtype, bf16 or
+    float32) then the rotation; see module docstring."""
+    return _direct(_QkNormRope, _qk_norm_rope_op, _qk_norm_rope_impl, (x, weight, eps, cos, sin),
+                   (x, weight, cos, sin))
+
+
 @torch.library.custom_op("avgen_amd::qk_norm_rope_bwd", mutates_args=())
+def _qk_norm_rope_bwd_op(
+    dy: torch.Tensor, x: torch.Tensor, weight: Optional[torch.Tensor], eps: float, cos: Optional[torch.Tensor],
+    sin: Optional[torch.Tensor],
+) -> tuple[torch.Tensor, torch.Tensor]:
+    """``(dx, dweight)`` of ``qk_norm_rope`` (``dweight`` fp32; zeros(0) without a gain)."""
+    return _qk_norm_rope_bwd(dy, x, weight, eps, cos, sin)
+
+
+def _qk_norm_rope_bwd(dy, x, weight, eps, cos, sin):
+    dx, dw = _qk_norm_rope_bwd_impl(dy, x, weight, eps, cos, sin)
+    return dx, (dw if dw is not None else x.new_zeros(0, dtype=torch.float32))
+
+
 def qk_norm_rope_bwd(
     dy: torch.Tensor, x: torch.Tensor, weight: Optional[torch.Tensor], eps: float, cos: Optional[torch.Tensor],
     sin: Optional[torch.Tensor],
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """``(dx, dweight)`` of ``qk_norm_rope`` (``dweight`` fp32; zeros(0) without a gain)."""
-    dx, dw = _qk_norm_rope_bwd_impl(dy, x, weight, eps, cos, sin)
-    return dx, (dw if dw is not None else x.new_zeros(0, dtype=torch.float32))
+    if _grad_direct(dy, x, weight, cos, sin):
+        return _qk_norm_rope_bwd(dy, x, weight, eps, cos, sin)
+    return _qk_norm_rope_bwd_op(dy, x, weight, eps, cos, sin)
 
 
-@qk_norm_rope_bwd.register_fake
+@_qk_norm_rope_bwd_op.register_fake
 def _(dy, x, weight, eps, cos, sin):
     return torch.empty_like(x), x.new_empty(0 if weight is None else x.shape[-1], dtype=torch.float32)
 
@@ -1246,6 +1425,16 @@ def _qk_norm_backward(ctx, dy):
 
 
 torch.library.register_autograd("avgen_amd::qk_norm_rope", _qk_norm_backward, setup_context=_qk_norm_setup)
+
+
+class _QkNormRope(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, *args):
+        result = _qk_norm_rope_impl(*args)
+        _qk_norm_setup(ctx, args, result)
+        return result
+
+    backward = staticmethod(_qk_norm_backward)
 
 
 def _fwd_setup(ctx, inputs, output):
@@ -1270,6 +1459,19 @@ def _fwd_backward(ctx, dout, _dlse):
 torch.library.register_autograd("avgen_amd::flash_fwd", _fwd_backward, setup_context=_fwd_setup)
 
 
+class _FlashFwd(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, *args):
+        result = _fwd_impl(*args)
+        ctx.set_materialize_grads(False)
+        _fwd_setup(ctx, args, result)
+        return result
+
+    @staticmethod
+    def backward(ctx, dout, _dlse):
+        return (None,) * 7 if dout is None else _fwd_backward(ctx, dout, None)
+
+
 def _rope_setup(ctx, inputs, output):
     _x, cos, sin, inverse = inputs
     ctx.inverse = inverse
@@ -1282,6 +1484,16 @@ def _rope_backward(ctx, grad):
 
 
 torch.library.register_autograd("avgen_amd::rope_apply", _rope_backward, setup_context=_rope_setup)
+
+
+class _RopeApply(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, *args):
+        result = _rope_apply_impl(*args)
+        _rope_setup(ctx, args, result)
+        return result
+
+    backward = staticmethod(_rope_backward)
 
 
 # ---------------------------------------------------------------------------

@@ -291,10 +291,10 @@ def _ring_forward_fused(query, key, value, key_mask, cp, scale, tables_q, tables
     lse = torch.empty((B, Hq, Lq), dtype=torch.float32, device=query.device)
     out = ops._kernel_ready(torch.empty_like(query, memory_format=torch.preserve_format))
     for r, (a, b) in enumerate(bounds):
-        ops.ring_fwd_step_(query, key[:, :, a:b], value[:, :, a:b],
-                           None if key_mask is None else key_mask[:, a:b], tables_q,
-                           _chunk_tables(tables_k, a, b), scale, acc, lse, out,
-                           first=r == 0, last=r == cp - 1)
+        tk = _chunk_tables(tables_k, a, b)
+        ops._ring_fwd_step_impl(query, key[:, :, a:b], value[:, :, a:b],
+                                None if key_mask is None else key_mask[:, a:b], tables_q.cos, tables_q.sin,
+                                tk.cos, tk.sin, scale, acc, lse, out, r == 0, r == cp - 1)
     return out, lse
 
 
@@ -317,10 +317,11 @@ def _ring_backward_fused(grad_out, query, key, value, out, lse, key_mask, cp, sc
     bounds = [shard_bounds(L, cp, r) for r in range(cp)]
     ws = _ring_workspace(B, Hq, Hkv, Lq, D, bounds, query.device)
     for r, (a, b) in enumerate(bounds):
-        ops.ring_bwd_step(grad_out, query, key[:, :, a:b], value[:, :, a:b], out, lse,
-                          None if key_mask is None else key_mask[:, a:b], tables_q, _chunk_tables(tables_k, a, b),
-                          scale, dq_acc, dk[:, :, a:b], dv[:, :, a:b], workspace=ws, reuse_query_side=r > 0)
-    ops.ring_dq_finish(dq_acc, tables_q, dq)
+        tk = _chunk_tables(tables_k, a, b)
+        ops._ring_bwd_step_impl(grad_out, query, key[:, :, a:b], value[:, :, a:b], out, lse,
+                                None if key_mask is None else key_mask[:, a:b], tables_q.cos, tables_q.sin, tk.cos,
+                                tk.sin, scale, dq_acc, dk[:, :, a:b], dv[:, :, a:b], ws, r > 0)
+    ops._ring_dq_finish_impl(dq_acc, tables_q.cos, tables_q.sin, dq)
     return dq, dk, dv
 
 
@@ -335,6 +336,10 @@ def _ring_attention_rope_op(
     query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, key_mask: Optional[torch.Tensor],
     cos_q: torch.Tensor, sin_q: torch.Tensor, cos_k: torch.Tensor, sin_k: torch.Tensor, cp: int, scale: float,
 ) -> tuple[torch.Tensor, torch.Tensor]:
+    return _ring_rope_fwd(query, key, value, key_mask, cos_q, sin_q, cos_k, sin_k, cp, scale)
+
+
+def _ring_rope_fwd(query, key, value, key_mask, cos_q, sin_q, cos_k, sin_k, cp, scale):
     return _ring_forward_fused(query, key, value, key_mask, cp, scale, RotaryTables(cos_q, sin_q),
                                RotaryTables(cos_k, sin_k))
 
@@ -351,8 +356,7 @@ def _ring_attention_rope_bwd_op(
     lse: torch.Tensor, key_mask: Optional[torch.Tensor], cos_q: torch.Tensor, sin_q: torch.Tensor,
     cos_k: torch.Tensor, sin_k: torch.Tensor, cp: int, scale: float,
 ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    return _ring_backward_fused(grad_out.contiguous(), query, key, value, out, lse, key_mask, cp, scale,
-                                RotaryTables(cos_q, sin_q), RotaryTables(cos_k, sin_k))
+    return _ring_rope_bwd(grad_out, query, key, value, out, lse, key_mask, cos_q, sin_q, cos_k, sin_k, cp, scale)
 
 
 @_ring_attention_rope_bwd_op.register_fake
@@ -369,15 +373,35 @@ def _ring_rope_setup(ctx, inputs, output):
     ctx.mark_non_differentiable(lse)
 
 
+def _ring_rope_bwd(grad_out, query, key, value, out, lse, key_mask, cos_q, sin_q, cos_k, sin_k, cp, scale):
+    return _ring_backward_fused(grad_out.contiguous(), query, key, value, out, lse, key_mask, cp, scale,
+                                RotaryTables(cos_q, sin_q), RotaryTables(cos_k, sin_k))
+
+
 def _ring_rope_backward(ctx, grad_out, _grad_lse):
     query, key, value, out, lse, key_mask, cos_q, sin_q, cos_k, sin_k = ctx.saved_tensors
-    dq, dk, dv = _ring_attention_rope_bwd_op(grad_out, query, key, value, out, lse, key_mask, cos_q, sin_q, cos_k,
-                                             sin_k, ctx.cp, ctx.scale)
+    bwd = _ring_rope_bwd if ops._grad_direct(grad_out, *ctx.saved_tensors) else _ring_attention_rope_bwd_op
+    dq, dk, dv = bwd(grad_out, query, key, value, out, lse, key_mask, cos_q, sin_q, cos_k, sin_k, ctx.cp, ctx.scale)
     return dq, dk, dv, None, None, None, None, None, None, None
 
 
 torch.library.register_autograd("avgen_amd::ring_attention_rope", _ring_rope_backward,
                                 setup_context=_ring_rope_setup)
+
+
+class _RingAttentionRope(torch.autograd.Function):
+    """The op pair above for plain eager calls (see ``ops._plain_eager``)."""
+
+    @staticmethod
+    def forward(ctx, *args):
+        result = _ring_rope_fwd(*args)
+        ctx.set_materialize_grads(False)
+        _ring_rope_setup(ctx, args, result)
+        return result
+
+    @staticmethod
+    def backward(ctx, grad_out, _grad_lse):
+        return (None,) * 10 if grad_out is None else _ring_rope_backward(ctx, grad_out, None)
 
 
 class _RingAttention(torch.autograd.Function):
@@ -449,6 +473,6 @@ def ring_attention(
             return _RingAttention.apply(apply_rotary(query, tables_q), apply_rotary(key, tables_k), value, key_mask,
                                         cp, scale)
         s = ops.default_scale(query.shape[-1]) if scale is None else float(scale)
-        return _ring_attention_rope_op(query, key, value, key_mask, tables_q.cos, tables_q.sin, tables_k.cos,
-                                       tables_k.sin, int(cp), s)
+        tensors = (query, key, value, key_mask, tables_q.cos, tables_q.sin, tables_k.cos, tables_k.sin)
+        return ops._direct(_RingAttentionRope, _ring_attention_rope_op, _ring_rope_fwd, (*tensors, int(cp), s), tensors)
     return _RingAttention.apply(query, key, value, key_mask, cp, scale)
