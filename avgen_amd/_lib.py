@@ -196,6 +196,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ),
     "avattn_bwd_f32_workspace_size": (c_size, [c_i32, c_i32, c_i32]),
     "avattn_bwd_f32_staged_workspace_size": (c_size, [c_i32, c_i32, c_i32, c_i32, c_i32, c_i32]),
+    "avattn_bwd_f32_split_workspace_size": (c_size, [c_i32] * 6),
     "avattn_bwd_f32": (
         ctypes.c_int,
         [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr,
@@ -218,6 +219,18 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
          c_ptr,
          c_ptr],
     ),
+    "avattn_fwd_f32_split": (
+        ctypes.c_int,
+        [c_ptr, c_ptr, c_ptr, c_i64p, c_i64p, c_i64p,
+         c_i32, c_i32, c_i32, c_i32, c_i32, c_i32,
+         c_ptr, c_i64,
+         c_ptr, c_ptr, c_i64,
+         c_f32,
+         c_ptr, c_i64p, c_ptr,
+         c_ptr, c_size,
+         c_ptr],
+    ),
+    "avattn_fwd_f32_split_workspace_size": (c_size, [c_i32] * 5),
     "avattn_bwd_windowed_f32": (
         ctypes.c_int,
         [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr,

@@ -62,7 +62,21 @@ struct F32Args {
   // [wlo[b*wsb + r], whi[b*wsb + r]), clamped into 0 <= lo <= hi <= Lk
   const int32_t *wlo, *whi;
   int64_t wsb;
+  // split of the grid's partial last round (nsplit 0: none): its last nsplit
+  // row (forward) or key (dK/dV) blocks go to nparts workgroups each, one per
+  // range of tiles, which leave partial sums in part
+  float* part;
+  int nsplit, nparts;
+  int nblocks;  // dK/dV: 128-key blocks of this pass
 };
+
+// The block a workgroup takes of a grid of `total` blocks whose last nsplit
+// are split, and which part of it (-1: all).
+__device__ __forceinline__ void split_block(const F32Args& a, int total, int& bid, int& part) {
+  const int nfull = total - a.nsplit, i = (int)blockIdx.x - nfull;
+  bid = i < 0 ? (int)blockIdx.x : nfull + i / a.nparts;
+  part = i < 0 ? -1 : i % a.nparts;
+}
 
 __device__ __forceinline__ f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 __device__ __forceinline__ void st4(float* p, const f32x4& v) { *reinterpret_cast<f32x4*>(p) = v; }
@@ -104,6 +118,26 @@ __device__ __forceinline__ bool rows_meet_block(const F32Args& a, int lo, int hi
   return __builtin_amdgcn_ballot_w64(use && lo < k1 && hi > k0) != 0;
 }
 
+// Writes a query row from its accumulators (o[dt] register i: channel 32*dt +
+// 8*(i/4) + 4*(l/32) + i%4), maximum m and sum l over all its keys.  l > 0:
+// normal row; l == 0: no valid key (out 0, lse -inf); NaN: a NaN or +inf
+// score reached the row.
+template <int D>
+__device__ __forceinline__ void write_row_f32(const F32Args& a, const f32x16 (&o)[D / 32], float m, float l, int bh,
+                                              int row) {
+  const int hh = (threadIdx.x >> 5) & 1;
+  const float nan = __builtin_nanf("");
+  const float inv = l > 0.f ? 1.f / l : (l == 0.f ? 0.f : nan);
+  float* op = a.o + bh / a.Hq * a.osb + bh % a.Hq * a.osh + (int64_t)row * a.osl;
+#pragma unroll
+  for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      st4(op + 32 * dt + 8 * g + 4 * hh,
+          f32x4{o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv, o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv});
+  if (hh == 0) a.lse[(int64_t)bh * a.Lq + row] = l > 0.f ? fmaf(m, a.scale, logf(l)) : (l == 0.f ? kNegInf : nan);
+}
+
 // ---------------------------------------------------------------------------
 // Forward
 // ---------------------------------------------------------------------------
@@ -139,7 +173,10 @@ __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(F32Args a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
   const int nqb = (a.Lq + ROWS - 1) / ROWS;
-  const int qb = blockIdx.x % nqb, bh = blockIdx.x / nqb;
+  const int total = nqb * a.B * a.Hq;
+  int bid, part;
+  split_block(a, total, bid, part);
+  const int qb = bid % nqb, bh = bid / nqb;
   const int b = bh / a.Hq, h = bh % a.Hq, hk = h / (a.Hq / a.Hkv);
   const int row = qb * ROWS + wave * 32 + l32;
   const bool valid = row < a.Lq;
@@ -203,6 +240,11 @@ __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(F32Args a) {
     __shared__ int red[8];
     if (valid) row_window(a, b, row, wl, wh);
     window_tiles<4>(wl, wh, valid, red, t0, ntile);
+  }
+  if (part >= 0) {  // this part's share of the tiles (possibly none)
+    const int n = ntile - t0;
+    ntile = t0 + n * (part + 1) / a.nparts;
+    t0 += n * part / a.nparts;
   }
   if (t0 < ntile) {
     fetch(t0 * KT);
@@ -278,21 +320,56 @@ __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(F32Args a) {
     if (t + 1 < ntile) store(buf ^ 1);
   }
 
-  // The row sum over both halves of the keys; l > 0: normal row; l == 0: no
-  // valid key (out 0, lse -inf); NaN: a NaN or +inf score reached the row.
   l = halves_sum(l);
-  if (!valid) return;
-  const float nan = __builtin_nanf("");
-  const float inv = l > 0.f ? 1.f / l : (l == 0.f ? 0.f : nan);
-  float* op = a.o + b * a.osb + h * a.osh + (int64_t)row * a.osl;
-  // o[dt] register i: channel 32*dt + 8*(i/4) + 4*hh + i%4 of this lane's query
+  if (part >= 0) {
+    // One part of split rows: raw accumulators, maximum and sum, in the lane
+    // order fwd_f32_combine_kernel reads them in.
+    float* slot = a.part + (((int64_t)(bid - total + a.nsplit) * a.nparts + part) * 4 + wave) * fwd_slot_floats(32, D);
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
-      st4(op + 32 * dt + 8 * g + 4 * hh,
-          f32x4{o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv, o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv});
-  if (hh == 0) a.lse[(int64_t)bh * a.Lq + row] = l > 0.f ? fmaf(m, a.scale, logf(l)) : (l == 0.f ? kNegInf : nan);
+      for (int g = 0; g < 4; ++g)
+        st4(slot + ((dt * 4 + g) * 64 + lane) * 4,
+            f32x4{o[dt][4 * g], o[dt][4 * g + 1], o[dt][4 * g + 2], o[dt][4 * g + 3]});
+    if (hh == 0) slot[32 * D + l32] = m, slot[32 * D + 32 + l32] = l;
+    return;
+  }
+  if (valid) write_row_f32<D>(a, o, m, l, bh, row);
+}
+
+// The split row blocks: one wave per 32 rows adds the parts in order, each
+// scaled from its own maximum to the largest, and writes the rows.
+template <int D>
+__global__ __launch_bounds__(64) void fwd_f32_combine_kernel(F32Args a) {
+  constexpr int DT = D / 32, SLOT = fwd_slot_floats(32, D);
+  const int lane = threadIdx.x, l32 = lane & 31;
+  const int sb = blockIdx.x / 4, wave = blockIdx.x % 4;
+  const int nqb = (a.Lq + 127) / 128;
+  const int bid = nqb * a.B * a.Hq - a.nsplit + sb;
+  const float* slot = a.part + ((int64_t)sb * a.nparts * 4 + wave) * SLOT;
+  float m = kNegInf;
+  for (int p = 0; p < a.nparts; ++p) m = fmaxf(m, slot[(int64_t)p * 4 * SLOT + 32 * D + l32]);
+  f32x16 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) o[dt] = zero16();
+  float l = 0.f;
+  for (int p = 0; p < a.nparts; ++p) {
+    const float* sp = slot + (int64_t)p * 4 * SLOT;
+    const float mp = sp[32 * D + l32];
+    // no attended key in this part (mp -inf): nothing, unless a NaN reached it
+    const float w = mp == kNegInf ? 0.f : __builtin_amdgcn_exp2f((mp - m) * a.c);
+    l = fmaf(sp[32 * D + 32 + l32], w, l);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 x = ld4(sp + ((dt * 4 + g) * 64 + lane) * 4);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[dt][4 * g + r] = fmaf(x[r], w, o[dt][4 * g + r]);
+      }
+  }
+  const int row = bid % nqb * 128 + wave * 32 + l32;
+  if (row < a.Lq) write_row_f32<D>(a, o, m, l, bid / nqb, row);
 }
 
 // Zeros to out and -inf to lse (no keys at all).
@@ -349,17 +426,17 @@ __device__ __forceinline__ void load_row_ksteps(float (&r)[D / 2], const float* 
     for (int e = 0; e < DT; ++e) r[DT * u + e] = in ? p[32 * e + u + 16 * hh] : 0.f;
 }
 
-// Staging of one 32-row tile in that layout by 512 threads: thread slot v =
-// tid + 512*i holds row v/32, channels 32*t + v%32.
-template <int D>
+// Staging of one 32-row tile in that layout by NT threads: thread slot v =
+// tid + NT*i holds row v/32, channels 32*t + v%32.
+template <int D, int NT = 512>
 struct Tile32 {
-  static constexpr int DT = D / 32, PITCH = D + 4, SL = 32 * 32 / 512;
+  static constexpr int DT = D / 32, PITCH = D + 4, SL = 32 * 32 / NT;
   using vdt = float __attribute__((ext_vector_type(DT)));
   float x[SL][DT];
   __device__ __forceinline__ void fetch(const float* base, int64_t rs, int r0, int n, int tid) {
 #pragma unroll
     for (int i = 0; i < SL; ++i) {
-      const int v = tid + 512 * i, row = r0 + v / 32;
+      const int v = tid + NT * i, row = r0 + v / 32;
       const float* p = base + (int64_t)row * rs + (v % 32);
 #pragma unroll
       for (int t = 0; t < DT; ++t) x[i][t] = row < n ? p[32 * t] : 0.f;
@@ -368,7 +445,7 @@ struct Tile32 {
   __device__ __forceinline__ void store(float* tile, int tid) const {
 #pragma unroll
     for (int i = 0; i < SL; ++i) {
-      const int v = tid + 512 * i;
+      const int v = tid + NT * i;
       vdt y;
 #pragma unroll
       for (int t = 0; t < DT; ++t) y[t] = x[i][t];
@@ -406,7 +483,9 @@ __global__ __launch_bounds__(512) void bwd_dkdv_f32_kernel(F32Args a) {
   const int l32 = lane & 31, hh = lane >> 5;
   const int pair = wave & 3, role = wave >> 2;  // role 0: P wave, 1: dS wave
   const int nkb = (a.Lk + KPB - 1) / KPB;
-  const int kb = blockIdx.x % nkb, bhk = a.pair0 + blockIdx.x / nkb;
+  int bid, part;
+  split_block(a, a.nblocks, bid, part);
+  const int kb = bid % nkb, bhk = a.pair0 + bid / nkb;
   const int b = bhk / a.Hkv, hk = bhk % a.Hkv;
   const int group = a.Hq / a.Hkv;
   const int k0 = kb * KPB + pair * 32;  // the pair's first key
@@ -476,6 +555,11 @@ __global__ __launch_bounds__(512) void bwd_dkdv_f32_kernel(F32Args a) {
     }
     tb = __builtin_amdgcn_readfirstlane(r1 / QT);
     ntile = __builtin_amdgcn_readfirstlane(lo > r1 ? (lo + QT - 1) / QT : r1 / QT);
+  }
+  if (part >= 0) {  // this part's share of every query head's tiles (possibly none)
+    const int n = ntile - tb;
+    ntile = tb + n * (part + 1) / a.nparts;
+    tb += n * part / a.nparts;
   }
   for (int gi = 0; gi < group; ++gi) {
     const int h = hk * group + gi;
@@ -551,6 +635,18 @@ __global__ __launch_bounds__(512) void bwd_dkdv_f32_kernel(F32Args a) {
     __syncthreads();  // P of the last tile handed over
     if (role == 1 && ntile > tb) ds_step(s, ntile - 1, gi);
   }
+  if (part >= 0) {
+    // Unscaled partial sums, [dV, dK][128 keys][D]; dkv_f32_reduce_kernel
+    // adds the parts and zeroes masked keys.
+    float* pp = a.part + (((int64_t)(bid - a.nblocks + a.nsplit) * a.nparts + part) * 2 + role) * KPB * D;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float* gp = pp + (pair * 32 + 8 * (i / 4) + 4 * hh + (i % 4)) * D + l32;
+#pragma unroll
+      for (int d = 0; d < DT; ++d) gp[32 * d] = acc[d][i];
+    }
+    return;
+  }
   // acc[d] register i: key k0 + 8*(i/4) + 4*hh + i%4, channel 32*d + l32.
   // Masked keys: exactly zero (their P is 0; a non-finite dO or V elsewhere
   // in the row must not reach them through 0 * inf).
@@ -566,6 +662,30 @@ __global__ __launch_bounds__(512) void bwd_dkdv_f32_kernel(F32Args a) {
 #pragma unroll
     for (int d = 0; d < DT; ++d) gp[32 * d] = ok ? acc[d][i] * f : 0.f;
   }
+}
+
+// dK and dV of the split key blocks: one thread per (block, dV or dK, key, 4
+// channels) adds the parts in order.
+template <int D>
+__global__ __launch_bounds__(256) void dkv_f32_reduce_kernel(F32Args a) {
+  constexpr int KPB = 128, CQ = D / 4;
+  const int u = blockIdx.x * 256 + threadIdx.x;
+  const int c = u % CQ, r = u / CQ % KPB, role = u / (CQ * KPB) % 2, sb = u / (CQ * KPB * 2);
+  if (sb >= a.nsplit) return;
+  const int nkb = (a.Lk + KPB - 1) / KPB;
+  const int bid = a.nblocks - a.nsplit + sb;
+  const int bhk = a.pair0 + bid / nkb;
+  const int b = bhk / a.Hkv, hk = bhk % a.Hkv;
+  const int key = bid % nkb * KPB + r;
+  if (key >= a.Lk) return;
+  f32x4 t = {0.f, 0.f, 0.f, 0.f};
+  for (int p = 0; p < a.nparts; ++p)
+    t += ld4(a.part + ((((int64_t)sb * a.nparts + p) * 2 + role) * KPB + r) * D + 4 * c);
+  const float f = role == 0 ? 1.f : a.scale;
+  t = key_ok(a, b, key) ? f32x4{t[0] * f, t[1] * f, t[2] * f, t[3] * f} : f32x4{0.f, 0.f, 0.f, 0.f};
+  float* gb = role == 0 ? a.dv + b * a.dvsb + hk * a.dvsh + (int64_t)key * a.dvsl
+                        : a.dk + b * a.dksb + hk * a.dksh + (int64_t)key * a.dksl;
+  st4(gb + 4 * c, t);
 }
 
 // dQ on the fp32 matrix cores: per 32 query rows a pair of waves on one
@@ -706,8 +826,9 @@ __global__ __launch_bounds__(512) void bwd_dq_f32_kernel(F32Args a) {
   }
 }
 
-// dQ = scale * dS K from the staged dS: eight waves per workgroup, 32 query
-// rows each, 32-key tiles of K in LDS (the backward tile layout).  A lane
+// dQ = scale * dS K from the staged dS: four waves per workgroup, 32 query
+// rows each (two or more workgroups per CU fill a short last round better
+// than one of eight waves did), 32-key tiles of K in LDS (the backward tile layout).  A lane
 // reads its row's dS over keys 16*(l/32) .. +15 of a tile (64 contiguous
 // bytes of the tile's 32x32 block) straight into registers, a tile ahead;
 // k-step j contracts keys j and 16 + j, so one LDS read gives the lane its
@@ -715,8 +836,8 @@ __global__ __launch_bounds__(512) void bwd_dq_f32_kernel(F32Args a) {
 // the tiles meeting its rows' windows, and a wave multiplies only the key
 // blocks its rows meet (the blocks the windowed dK/dV kernel wrote).
 template <int D, bool WIN>
-__global__ __launch_bounds__(512) void bwd_dq_ds_f32_kernel(F32Args a) {
-  constexpr int KT = 32, ROWS = 256, PITCH = D + 4, DT = D / 32;
+__global__ __launch_bounds__(256, 2) void bwd_dq_ds_f32_kernel(F32Args a) {
+  constexpr int KT = 32, ROWS = 128, PITCH = D + 4, DT = D / 32;
   using vdt = float __attribute__((ext_vector_type(DT)));
   __shared__ __attribute__((aligned(16))) float ks[2][KT * PITCH];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -732,9 +853,9 @@ __global__ __launch_bounds__(512) void bwd_dq_ds_f32_kernel(F32Args a) {
   const bool valid = r0 + l32 < a.Lq;
   int wl = 0, wh = a.Lk, t0 = 0, ntile_w = ntile;
   if constexpr (WIN) {
-    __shared__ int red[16];
+    __shared__ int red[8];
     if (valid) row_window(a, b, r0 + l32, wl, wh);
-    window_tiles<8>(wl, wh, valid, red, t0, ntile_w);
+    window_tiles<4>(wl, wh, valid, red, t0, ntile_w);
   }
   // does this wave multiply key tile t
   auto takes = [&](int t) {
@@ -747,7 +868,7 @@ __global__ __launch_bounds__(512) void bwd_dq_ds_f32_kernel(F32Args a) {
 #pragma unroll
   for (int d = 0; d < DT; ++d) dq[d] = zero16();
   const float* kb = a.k + b * a.ksb + hk * a.ksh;
-  Tile32<D> sk;
+  Tile32<D, 256> sk;
   f32x4 pa[4];
   auto fetch = [&](int t) {
     sk.fetch(kb, a.ksl, t * KT, a.Lk, tid);
@@ -1025,10 +1146,41 @@ int check_f32_dims(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lq, int32_t Lk, i
 
 size_t r256(size_t x) { return (x + 255) / 256 * 256; }
 
+// Split of the forward's partial last round over ranges of 32-key tiles: the
+// number of parts (2..8, at least 4 tiles each) with the smallest estimated
+// time if it saves 4 us or more.  Two workgroups of 128 rows (three at
+// head_dim 64) share a CU and its matrix cores; with fewer there, each is
+// faster.  Times as measured on an MI355X at its full clock, which fp32
+// products hold.
+FwdSplit fwd_f32_split_plan(int B, int Hq, int Lq, int Lk, int D) {
+  constexpr int kCus = 256;
+  const int per_cu = D == 64 ? 3 : 2, slots = per_cu * kCus;
+  FwdSplit best{0, 0, 0};
+  const int ntile = (Lk + 31) / 32;
+  const int r = (int)((int64_t)((Lq + 127) / 128) * B * Hq % slots);
+  const float tile_us = D == 64 ? 5.2f : 7.f, fixed_us = 4.f;
+  auto rounds = [&](int n) {
+    const int k = (n % slots + kCus - 1) / kCus;
+    return n / slots + (k == 0 ? 0.f : (k + 0.2f * (per_cu - k)) / per_cu);
+  };
+  const float slot_bytes = 4.f * fwd_slot_floats(128, D);
+  float cost = rounds(r) * (ntile * tile_us + fixed_us) - 4.f;
+  for (int p = 2; p <= 8 && ntile / p >= 4; ++p) {
+    const float c = rounds(r * p) * (ntile * tile_us / p + fixed_us) + 5.f + r * p * slot_bytes * 0.5e-6f;
+    if (c < cost) {
+      cost = c;
+      best = FwdSplit{r, p, (size_t)r * p * fwd_slot_floats(128, D) * sizeof(float)};
+    }
+  }
+  return best;
+}
+
 template <int D, bool WIN>
 void launch_fwd_f32(const F32Args& a, hipStream_t s) {
-  const int nqb = (a.Lq + 127) / 128;
-  hipLaunchKernelGGL((fwd_f32_kernel<D, WIN>), dim3((unsigned)(nqb * a.B * a.Hq)), dim3(256), 0, s, a);
+  const int64_t blocks = (int64_t)((a.Lq + 127) / 128) * a.B * a.Hq;
+  const dim3 grid((unsigned)(blocks - a.nsplit + (int64_t)a.nsplit * a.nparts));
+  hipLaunchKernelGGL((fwd_f32_kernel<D, WIN>), grid, dim3(256), 0, s, a);
+  if (a.nsplit > 0) hipLaunchKernelGGL(fwd_f32_combine_kernel<D>, dim3(4 * a.nsplit), dim3(64), 0, s, a);
 }
 
 // Staged dS floats per (batch, kv head) pair (see F32Args::ds).
@@ -1036,8 +1188,19 @@ int64_t ds_floats_per_pair(int group, int Lq, int Lk) {
   return (int64_t)group * ((Lq + 31) / 32) * 32 * ((Lk + 127) / 128) * 128;
 }
 
+// Floats of one split dK/dV part.
+constexpr int dkv_f32_slot_floats(int D) { return 2 * 128 * D; }
+// The dK/dV split of a staged backward in one pass (one 128-key block per
+// workgroup and CU): the last round's blocks over ranges of query tiles.
+// (1,20,4096,128): 640 blocks, 2.5 rounds.
+FwdSplit dkv_f32_split_plan(int64_t blocks, int D) {
+  const TailSplit t = plan_tail_split(blocks, 256, kSplitSlots);
+  return FwdSplit{t.nsplit, t.nparts, (size_t)t.nsplit * t.nparts * dkv_f32_slot_floats(D) * sizeof(float)};
+}
+
 // pairs_per_pass 0: dQ recomputes S and dP; else dS is staged for that many
-// (batch, kv head) pairs at a time.
+// (batch, kv head) pairs at a time.  With a.part the (single) pass's dK/dV is
+// split.
 template <int D, bool WIN>
 void launch_bwd_f32(F32Args a, int pairs_per_pass, hipStream_t s) {
   const int64_t rows = (int64_t)a.B * a.Hq * a.Lq;
@@ -1046,17 +1209,25 @@ void launch_bwd_f32(F32Args a, int pairs_per_pass, hipStream_t s) {
   const int pairs = a.B * a.Hkv;
   if (pairs_per_pass == 0) {
     a.pair0 = 0;
-    hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, false, WIN>), dim3((unsigned)(nkb * pairs)), dim3(512), 0, s, a);
+    a.nblocks = nkb * pairs;
+    hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, false, WIN>), dim3((unsigned)a.nblocks), dim3(512), 0, s, a);
     const int nqb = (a.Lq + 127) / 128;
     hipLaunchKernelGGL((bwd_dq_f32_kernel<D, WIN>), dim3((unsigned)(nqb * a.B * a.Hq)), dim3(512), 0, s, a);
     return;
   }
-  const int group = a.Hq / a.Hkv, nrb = (a.Lq + 255) / 256;
+  const int group = a.Hq / a.Hkv, nrb = (a.Lq + 127) / 128;
   for (int p0 = 0; p0 < pairs; p0 += pairs_per_pass) {
     const int np = pairs - p0 < pairs_per_pass ? pairs - p0 : pairs_per_pass;
     a.pair0 = p0;
-    hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, true, WIN>), dim3((unsigned)(nkb * np)), dim3(512), 0, s, a);
-    hipLaunchKernelGGL((bwd_dq_ds_f32_kernel<D, WIN>), dim3((unsigned)(nrb * np * group)), dim3(512), 0, s, a);
+    a.nblocks = nkb * np;
+    const FwdSplit sp = a.part ? dkv_f32_split_plan(a.nblocks, D) : FwdSplit{0, 0, 0};
+    a.nsplit = sp.nsplit, a.nparts = sp.nparts;
+    const dim3 grid((unsigned)(a.nblocks - a.nsplit + a.nsplit * a.nparts));
+    hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, true, WIN>), grid, dim3(512), 0, s, a);
+    if (a.nsplit > 0)
+      hipLaunchKernelGGL(dkv_f32_reduce_kernel<D>, dim3((unsigned)(a.nsplit * (2 * 128 * (D / 4) / 256))), dim3(256), 0,
+                         s, a);
+    hipLaunchKernelGGL((bwd_dq_ds_f32_kernel<D, WIN>), dim3((unsigned)(nrb * np * group)), dim3(256), 0, s, a);
   }
 }
 
@@ -1082,7 +1253,7 @@ static int fwd_f32_entry(const float* q, const float* k, const float* v, const i
                          int32_t heads_kv, int32_t len_q, int32_t len_k, int32_t head_dim, const uint8_t* key_mask,
                          int64_t key_mask_batch_stride, const int32_t* window_lo, const int32_t* window_hi,
                          int64_t window_batch_stride, float scale, float* out, const int64_t* out_strides,
-                         float* lse, avattn_stream_t stream) {
+                         float* lse, avattn_stream_t stream, void* workspace = nullptr, size_t workspace_bytes = 0) {
   int st = check_f32_dims(batch, heads_q, heads_kv, len_q, len_k, head_dim);
   if (st != AVATTN_OK) return st;
   st = check_f32_windows(window_lo, window_hi, window_batch_stride, len_q);
@@ -1111,6 +1282,12 @@ static int fwd_f32_entry(const float* q, const float* k, const float* v, const i
   if (key_mask && key_mask_batch_stride != 0 && key_mask_batch_stride < len_k) return AVATTN_ERR_ARGUMENT;
   a.scale = scale, a.c = scale * kLog2e;
   a.wlo = window_lo, a.whi = window_hi, a.wsb = window_batch_stride;
+  const FwdSplit sp = fwd_f32_split_plan(batch, heads_q, len_q, len_k, head_dim);
+  if (workspace && sp.nsplit > 0 && workspace_bytes >= sp.bytes) {
+    if (!al16(workspace)) return AVATTN_ERR_WORKSPACE;
+    a.part = static_cast<float*>(workspace);
+    a.nsplit = sp.nsplit, a.nparts = sp.nparts;
+  }
   if (window_lo) {
     if (head_dim == 128)
       launch_fwd_f32<128, true>(a, s);
@@ -1144,6 +1321,23 @@ int avattn_fwd_windowed_f32(const float* q, const float* k, const float* v, cons
                        out_strides, lse, stream);
 }
 
+int avattn_fwd_f32_split(const float* q, const float* k, const float* v, const int64_t* q_strides,
+                         const int64_t* k_strides, const int64_t* v_strides, int32_t batch, int32_t heads_q,
+                         int32_t heads_kv, int32_t len_q, int32_t len_k, int32_t head_dim, const uint8_t* key_mask,
+                         int64_t key_mask_batch_stride, const int32_t* window_lo, const int32_t* window_hi,
+                         int64_t window_batch_stride, float scale, float* out, const int64_t* out_strides, float* lse,
+                         void* workspace, size_t workspace_bytes, avattn_stream_t stream) {
+  return fwd_f32_entry(q, k, v, q_strides, k_strides, v_strides, batch, heads_q, heads_kv, len_q, len_k, head_dim,
+                       key_mask, key_mask_batch_stride, window_lo, window_hi, window_batch_stride, scale, out,
+                       out_strides, lse, stream, workspace, workspace_bytes);
+}
+
+size_t avattn_fwd_f32_split_workspace_size(int32_t batch, int32_t heads_q, int32_t len_q, int32_t len_k,
+                                           int32_t head_dim) {
+  if (batch <= 0 || heads_q <= 0 || len_q <= 0 || len_k <= 0 || (head_dim != 64 && head_dim != 128)) return 0;
+  return fwd_f32_split_plan(batch, heads_q, len_q, len_k, head_dim).bytes;
+}
+
 size_t avattn_bwd_f32_workspace_size(int32_t batch, int32_t heads_q, int32_t len_q) {
   if (batch <= 0 || heads_q <= 0 || len_q <= 0) return 0;
   return 2 * r256((size_t)batch * heads_q * len_q * sizeof(float));
@@ -1157,6 +1351,15 @@ size_t avattn_bwd_f32_staged_workspace_size(int32_t batch, int32_t heads_q, int3
   const int64_t pp = kv_pairs_per_pass < pairs ? kv_pairs_per_pass : pairs;
   return (base + 4095) / 4096 * 4096 +
          (size_t)pp * (size_t)ds_floats_per_pair(heads_q / heads_kv, len_q, len_k) * sizeof(float);
+}
+
+size_t avattn_bwd_f32_split_workspace_size(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t len_q,
+                                           int32_t len_k, int32_t head_dim) {
+  if (check_f32_dims(batch, heads_q, heads_kv, len_q, len_k, head_dim) != AVATTN_OK) return 0;
+  if ((int64_t)batch * heads_q * len_q == 0 || len_k == 0) return 0;
+  const int64_t pairs = (int64_t)batch * heads_kv;
+  return avattn_bwd_f32_staged_workspace_size(batch, heads_q, heads_kv, len_q, len_k, (int32_t)pairs) +
+         dkv_f32_split_plan(pairs * ((len_k + 127) / 128), head_dim).bytes;
 }
 
 static int bwd_f32_entry(const float* dout, const float* q, const float* k, const float* v, const float* out,
@@ -1237,6 +1440,11 @@ static int bwd_f32_entry(const float* dout, const float* q, const float* k, cons
       pp = (int)((pairs + npass - 1) / npass);
       a.ds = reinterpret_cast<float*>(static_cast<char*>(workspace) + off);
       a.dsp = (int64_t)(per / sizeof(float));
+      // One pass and room behind its dS: the parts of a split dK/dV round.
+      const size_t end = off + (size_t)pairs * per;
+      const FwdSplit sp = dkv_f32_split_plan(pairs * ((len_k + 127) / 128), head_dim);
+      if (pp == pairs && sp.nsplit > 0 && workspace_bytes >= end + sp.bytes)
+        a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + end);
     }
   }
   a.wlo = window_lo, a.whi = window_hi, a.wsb = window_batch_stride;

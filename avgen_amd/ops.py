@@ -273,8 +273,10 @@ def _fwd_impl(q, k, v, key_mask, rope_cos, rope_sin, scale):
 def _f32_ready(t: torch.Tensor) -> torch.Tensor:
     """float32 rows for the fp32 kernels: head_dim contiguous, 16-byte aligned
     row starts (strides a multiple of 4 elements)."""
-    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0
-    ok = ok and all(s % 4 == 0 or n == 1 for s, n in zip(t.stride()[:3], t.shape[:3]))
+    s0, s1, s2, s3 = t.stride()
+    ok = s3 == 1 and t.data_ptr() % 16 == 0
+    if ok and (s0 | s1 | s2) % 4:
+        ok = all(s % 4 == 0 or n == 1 for s, n in zip((s0, s1, s2), t.shape[:3]))
     return t if ok else t.contiguous()
 
 
@@ -288,39 +290,29 @@ def _fwd_f32_impl(name, q, k, v, key_mask, rope_cos, rope_sin, scale):
         raise ValueError(f"{name}: pass both rotary tables or neither")
     if rope_cos is not None:
         q = _rope_apply_impl(q, rope_cos, rope_sin, False)
-    q, k, v = _f32_ready(q), _f32_ready(k), _f32_ready(v)
-    mask, msb = _normalise_mask(name, key_mask, B, Lk)
-    out = _f32_ready(torch.empty_like(q, memory_format=torch.preserve_format))
-    lse = torch.empty((B, Hq, Lq), device=q.device, dtype=torch.float32)
-    st = _lib.load().avattn_fwd_f32(
-        _ptr(q), _ptr(k), _ptr(v), _strides3(q), _strides3(k), _strides3(v),
-        B, Hq, Hkv, Lq, Lk, D,
-        _ptr(mask), msb,
-        float(scale),
-        _ptr(out), _strides3(out), _ptr(lse),
-        _stream(q.device),
-    )
-    _lib.check(st, name)
-    return out, lse
+    return _fwd_f32_launch(name, q, k, v, None, None, 0, key_mask, scale)
 
 
-def _fwd_windowed_f32_impl(name, q, k, v, lo, hi, wsb, key_mask, scale):
-    """The float32 forward with per-row key windows
-    (``avattn_fwd_windowed_f32``); ``lo``/``hi``/``wsb`` as checked by
-    ``_check_windows``."""
+def _fwd_f32_launch(name, q, k, v, lo, hi, wsb, key_mask, scale):
+    """``avattn_fwd_f32_split``: the float32 forward, with key windows when
+    ``lo``/``hi``/``wsb`` (as checked by ``_check_windows``) are given."""
     B, Hq, Lq, D = q.shape
     Hkv, Lk = k.shape[1], k.shape[2]
     q, k, v = _f32_ready(q), _f32_ready(k), _f32_ready(v)
     mask, msb = _normalise_mask(name, key_mask, B, Lk)
     out = _f32_ready(torch.empty_like(q, memory_format=torch.preserve_format))
     lse = torch.empty((B, Hq, Lq), device=q.device, dtype=torch.float32)
-    st = _lib.load().avattn_fwd_windowed_f32(
+    lib = _lib.load()
+    need = lib.avattn_fwd_f32_split_workspace_size(B, Hq, Lq, Lk, D)
+    ws = _workspace(need, q.device) if need else None
+    st = lib.avattn_fwd_f32_split(
         _ptr(q), _ptr(k), _ptr(v), _strides3(q), _strides3(k), _strides3(v),
         B, Hq, Hkv, Lq, Lk, D,
         _ptr(mask), msb,
         _ptr(lo), _ptr(hi), wsb,
         float(scale),
         _ptr(out), _strides3(out), _ptr(lse),
+        _ptr(ws), need,
         _stream(q.device),
     )
     _lib.check(st, name)
@@ -347,7 +339,7 @@ def _bwd_f32_impl(name, dout, q, k, v, out, lse, key_mask, scale, windows=None):
     dk = _f32_ready(torch.empty_like(k))
     dv = _f32_ready(torch.empty_like(v))
     lib = _lib.load()
-    ws = _alloc_bwd_f32_workspace(B, Hq, Hkv, Lq, Lk, q.device)
+    ws = _alloc_bwd_f32_workspace(B, Hq, Hkv, Lq, Lk, q.device, D)
     head = (
         _ptr(dout), _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse),
         _strides3(dout), _strides3(q), _strides3(k), _strides3(v), _strides3(out),
@@ -376,12 +368,13 @@ def f32_ds_bytes_per_pair(group, Lq, Lk):
     return 4 * group * ((Lq + 31) // 32 * 32) * ((Lk + 127) // 128 * 128)
 
 
-def _alloc_bwd_f32_workspace(B, Hq, Hkv, Lq, Lk, device) -> torch.Tensor:
+def _alloc_bwd_f32_workspace(B, Hq, Hkv, Lq, Lk, device, D=None) -> torch.Tensor:
     """The float32 backward's workspace: with the staged-dS budget (the one
     the bf16 backward uses) holding at least one (batch, kv head) pair's fp32
     dS, the staged size for as many pairs per pass as fit in equal passes
-    (halving while the allocator cannot provide it), else the statistics
-    alone (dq recomputes S and dP)."""
+    (halving while the allocator cannot provide it; all of them in one pass
+    with ``D`` given: also room for a split last dK/dV round), else the
+    statistics alone (dq recomputes S and dP)."""
     lib = _lib.load()
     pairs = 0
     if B * Hkv > 0 and Lq > 0 and Lk > 0:
@@ -391,6 +384,8 @@ def _alloc_bwd_f32_workspace(B, Hq, Hkv, Lq, Lk, device) -> torch.Tensor:
         pairs = -(-(B * Hkv) // npass)
     while pairs > 0:
         try:
+            if D is not None and pairs == B * Hkv:
+                return _workspace(lib.avattn_bwd_f32_split_workspace_size(B, Hq, Hkv, Lq, Lk, D), device)
             return _workspace(lib.avattn_bwd_f32_staged_workspace_size(B, Hq, Hkv, Lq, Lk, int(pairs)), device)
         except torch.OutOfMemoryError:
             pairs = 0 if pairs == 1 else (pairs + 1) // 2
@@ -421,7 +416,7 @@ def _fwd_windowed_impl(q, k, v, window_lo, window_hi, key_mask, scale):
     Hkv, Lk = k.shape[1], k.shape[2]
     lo, hi, wsb = _check_windows(name, window_lo, window_hi, B, Lq)
     if q.dtype is torch.float32:
-        return _fwd_windowed_f32_impl(name, q, k, v, lo, hi, wsb, key_mask, scale)
+        return _fwd_f32_launch(name, q, k, v, lo, hi, wsb, key_mask, scale)
     q, k, v = _kernel_ready(q), _kernel_ready(k), _kernel_ready(v)
     mask, msb = _normalise_mask(name, key_mask, B, Lk)
     out = _kernel_ready(torch.empty_like(q, memory_format=torch.preserve_format))

@@ -684,6 +684,17 @@ size_t avattn_bwd_f32_staged_workspace_size(int32_t batch, int32_t heads_q, int3
                                             int32_t len_q, int32_t len_k,
                                             int32_t kv_pairs_per_pass);
 
+/*
+ * Workspace with which avattn_bwd_f32 / avattn_bwd_windowed_f32 stage dS for
+ * every (batch, kv head) pair at once and also split the last round of the
+ * dK/dV grid over ranges of queries where it is partial; dk and dv of the
+ * split keys differ from the unsplit ones in rounding only.  0 for a problem
+ * the backward would refuse or that is empty.
+ */
+size_t avattn_bwd_f32_split_workspace_size(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t len_q,
+                                           int32_t len_k, int32_t head_dim);
+
+
 int avattn_bwd_f32(const float* dout, const float* q, const float* k, const float* v,
                    const float* out, const float* lse,
                    const int64_t* dout_strides, const int64_t* q_strides,
@@ -725,6 +736,23 @@ int avattn_fwd_windowed_f32(const float* q, const float* k, const float* v,
                             float* out, const int64_t* out_strides,
                             float* lse,
                             avattn_stream_t stream);
+
+/*
+ * avattn_fwd_f32 / avattn_fwd_windowed_f32 (window_lo and window_hi NULL or
+ * both given) with a workspace for the parts of a split last round of the
+ * grid: avattn_fwd_f32_split_workspace_size() bytes (0: this shape is not
+ * split), 16-byte aligned.  With less (or NULL) the call runs unsplit; the
+ * split rows differ in rounding only.
+ */
+int avattn_fwd_f32_split(const float* q, const float* k, const float* v, const int64_t* q_strides,
+                         const int64_t* k_strides, const int64_t* v_strides, int32_t batch, int32_t heads_q,
+                         int32_t heads_kv, int32_t len_q, int32_t len_k, int32_t head_dim, const uint8_t* key_mask,
+                         int64_t key_mask_batch_stride, const int32_t* window_lo, const int32_t* window_hi,
+                         int64_t window_batch_stride, float scale, float* out, const int64_t* out_strides, float* lse,
+                         void* workspace, size_t workspace_bytes, avattn_stream_t stream);
+size_t avattn_fwd_f32_split_workspace_size(int32_t batch, int32_t heads_q, int32_t len_q, int32_t len_k,
+                                           int32_t head_dim);
+
 
 int avattn_bwd_windowed_f32(const float* dout, const float* q, const float* k, const float* v,
                             const float* out, const float* lse,
