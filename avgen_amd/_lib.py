@@ -78,6 +78,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "avattn_fp8_absmax_scales": (ctypes.c_int, [c_ptr, c_i64p, c_i32, c_i32, c_i32, c_i32, c_ptr, c_ptr]),
     "avattn_bwd_workspace_size": (c_size, [c_i32, c_i32, c_i32, c_i32, c_i32, c_i32]),
     "avattn_bwd_staged_workspace_size": (c_size, [c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32]),
+    "avattn_bwd_split_workspace_size": (c_size, [c_i32] * 6),
     "avattn_bwd_dq_staged": (
         ctypes.c_int,
         [c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, ctypes.c_float, c_ptr, c_i64p, c_ptr, c_size, ctypes.c_uint32,

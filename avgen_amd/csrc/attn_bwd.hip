@@ -106,13 +106,20 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
   const int nkt = (a.Lk + BK - 1) / BK;
   const int total = nkt * a.nkv;
   // Key blocks 0 .. nfull-1 take one workgroup each (query tiles all); the
-  // last a.nsplit blocks (the grid's partial last round) take a.nparts
-  // workgroups each, one per range of query tiles, whose fp32 partial
-  // dK/dV dkv_reduce_kernel sums.
+  // last a.nsplit blocks (the grid's partial last round, or all of them)
+  // take a.nparts workgroups each, one per range of query tiles, whose fp32
+  // partial dK/dV dkv_reduce_kernel sums.
   const int nfull = total - a.nsplit;
   int bid, part = -1;
-  if ((int)blockIdx.x < nfull) {
-    bid = xcd_remap(blockIdx.x, nfull);
+  if (nfull == 0) {
+    // A pair's key blocks of one part next to each other: they stream the
+    // same query tiles.
+    const int per = nkt * a.nparts;
+    const int u = xcd_remap_pairs(blockIdx.x, total * a.nparts, per, MASK);
+    bid = u / per * nkt + u % nkt;
+    part = u % per / nkt;
+  } else if ((int)blockIdx.x < nfull) {
+    bid = xcd_remap_pairs(blockIdx.x, nfull, nkt, MASK);
   } else {
     const int i = blockIdx.x - nfull;
     bid = nfull + i / a.nparts;
@@ -262,7 +269,10 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(BwdArgs a) {
   // A block outside the pair's hull of contributing tiles (every key masked):
   // dK and dV are zeros and dS is not read.
   if (MASK && STAGE && !WIN) {
-    if (2 * kt >= load_const_i32(a.khull, 2 * bhk + 1) || 2 * kt + 2 <= load_const_i32(a.khull, 2 * bhk)) ntq = 0;
+    if (2 * kt >= load_const_i32(a.khull, 2 * bhk + 1) || 2 * kt + 2 <= load_const_i32(a.khull, 2 * bhk)) {
+      if (part >= 0) return;  // the reduction reads no part of a masked key
+      ntq = 0;
+    }
   }
   if (part >= 0) {  // this part's share of the tiles (possibly none)
     const int p0 = ntq * part / a.nparts, p1 = ntq * (part + 1) / a.nparts;
@@ -749,7 +759,8 @@ __global__ __launch_bounds__(256) void dkv_reduce_kernel(BwdArgs a) {
   const int key = kt * BK + r;
   if (key >= a.Lk) return;
   f32x4 t = {0.f, 0.f, 0.f, 0.f};
-  for (int p = 0; p < a.nparts; ++p)
+  const bool attended = a.mask == nullptr || a.mask[b * a.msb + key] != 0;
+  for (int p = 0; attended && p < a.nparts; ++p)
     t += *reinterpret_cast<const f32x4*>(a.split_part + ((((int64_t)s * a.nparts + p) * 2 + role) * BK + r) * D + 4 * c);
   const float sc = role == 0 ? 1.f : a.scale;
   u32x2 w;
@@ -1152,7 +1163,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dq_ds_kernel(BwdArgs a) {
   const int nqg = a.Lqp / 32;
   const int nqb = (nqg + NW - 1) / NW;
   const int total = nqb * a.nkv * group;
-  const int bid = xcd_remap(blockIdx.x, total);
+  const int bid = xcd_remap_pairs(blockIdx.x, total, nqb * group, a.mask != nullptr);
   const int qb = bid % nqb;
   const int bq_rel = bid / nqb;             // (b, hq) within the pass
   const int bq = a.kv0 * group + bq_rel;    // b*Hq + hq
@@ -1338,6 +1349,39 @@ static int cu_count() {
   return n;
 }
 
+// Split of every key block of a short dK/dV grid (no windows) over 2..8 ranges
+// of query tiles (at least 8 each), or {0, 0}: for grids of at most one round,
+// and with a key mask of at most two, where blocks without an attended key
+// end at once and leave the rest unevenly spread (weighed as half of them).
+// Estimated from the time per 64-row tile and per workgroup and the parts'
+// traffic at 4 TB/s; a partial round clocks higher (see fwd_split_plan).
+// Backward: (1,16,20000,128) x 256 keys 498 -> 198 us, (1,20,10000) x 128 keys
+// 255 -> 104, (1,4,4096) self-attention 171 -> 150, 75,600 x 512 keys with
+// 388 and 0 attended (2 x 40 heads) 3.68 -> 2.86 ms; with 512 and 500
+// attended 5.28 -> 5.38.
+TailSplit dkv_split_plan(int64_t total, int tiles, int D, bool masked) {
+  constexpr int kCus = 256;
+  TailSplit best{0, 0};
+  if (total > (masked ? 2 * kCus : kCus)) return best;
+  const float work_us = tiles * (D == 64 ? 1.1f : 1.9f), fixed_us = 8.f;
+  auto rounds = [&](int64_t n) {
+    const int rem = (int)(n % kCus);
+    return n / kCus + (rem == 0 ? 0.f : 1.f - 0.38f * (1.f - (float)rem / kCus));
+  };
+  auto cost = [&](int64_t n, int p) {
+    return rounds(n * p) * (work_us / p + fixed_us) + (p > 1 ? 5.f + n * p * (1024.f * D) * 0.5e-6f : 0.f);
+  };
+  auto mean = [&](int p) { return masked ? 0.5f * (cost(total, p) + cost((total + 1) / 2, p)) : cost(total, p); };
+  float c = mean(1) - 4.f;
+  for (int p = 2; p <= 8 && tiles / p >= 8; ++p) {
+    if (mean(p) < c) {
+      c = mean(p);
+      best = TailSplit{(int)total, p};
+    }
+  }
+  return best;
+}
+
 template <int D>
 static void launch_dq_ds_d(const BwdArgs& a, hipStream_t stream) {
   const int group = a.Hq / a.Hkv;
@@ -1401,7 +1445,12 @@ static hipError_t launch_bwd_d(const BwdArgs& args, int kv_per_pass, hipStream_t
     // over several workgroups each (ranges of query tiles) so that the last
     // round is fuller and shorter.
     const int total = nkt * p.nkv;
-    const TailSplit ts = p.split_part ? plan_tail_split(total, cus, kSplitSlots) : TailSplit{0, 0};
+    TailSplit ts = p.split_part ? plan_tail_split(total, cus, kSplitSlots) : TailSplit{0, 0};
+    if (p.split_all != nullptr) {
+      // Every block split (the region holds the plan's parts).
+      ts = dkv_split_plan(total, (a.Lqp / 64) * (a.Hq / a.Hkv), D, mask);
+      p.split_part = p.split_all;
+    }
     p.nsplit = ts.nsplit;
     p.nparts = ts.nparts;
     {

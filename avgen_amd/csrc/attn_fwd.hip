@@ -185,7 +185,7 @@ __global__ __launch_bounds__(SMALL ? 256 : 512, SMALL ? 2 : 1) void attn_fwd_ker
   const int nfull = nqt * a.B * a.Hq - a.nsplit;
   int bid, part = -1;
   if ((int)blockIdx.x < nfull) {
-    bid = xcd_remap(blockIdx.x, nfull);
+    bid = xcd_remap_pairs(blockIdx.x, nfull, nqt * (a.Hq / a.Hkv), a.mask != nullptr);
   } else {
     const int i = blockIdx.x - nfull;
     bid = nfull + i / a.nparts;

@@ -388,6 +388,25 @@ size_t avattn_bwd_staged_workspace_size(int32_t batch, int32_t heads_q, int32_t 
   return staged_ds_offset(wl) + (size_t)n * ds_bytes_per_kv(heads_q / heads_kv, len_q, len_k);
 }
 
+namespace {
+// Bytes of the parts of a dK/dV grid with every block split (0: not split).
+size_t dkv_split_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lq, int32_t Lk, int32_t D, bool masked) {
+  const TailSplit t = dkv_split_plan((int64_t)B * Hkv * ((Lk + 127) / 128),
+                                     (int)(transpose_padded_len(Lq) / 64 * (Hq / Hkv)), D, masked);
+  return (size_t)t.nsplit * t.nparts * 256 * D * sizeof(float);
+}
+}  // namespace
+
+size_t avattn_bwd_split_workspace_size(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t len_q, int32_t len_k,
+                                       int32_t head_dim) {
+  if (check_bwd_dims(batch, heads_q, heads_kv, len_q, len_k, head_dim) != AVATTN_OK) return 0;
+  if ((int64_t)batch * heads_q * len_q == 0 || len_k == 0) return 0;
+  const size_t plain = dkv_split_bytes(batch, heads_q, heads_kv, len_q, len_k, head_dim, false);
+  const size_t masked = dkv_split_bytes(batch, heads_q, heads_kv, len_q, len_k, head_dim, true);
+  return avattn_bwd_staged_workspace_size(batch, heads_q, heads_kv, len_q, len_k, head_dim, batch * heads_kv) +
+         (plain > masked ? plain : masked);
+}
+
 // Compact staged-dS layout of a windowed backward (BwdArgs::ds_tab).
 struct CompactDs {
   const int32_t* table = nullptr;
@@ -546,6 +565,12 @@ static int bwd_impl(const void* dout, const void* q, const void* k, const void* 
     kv_per_pass = (int)(((size_t)a.nkv + npass - 1) / npass);
     a.ds = reinterpret_cast<bf16*>(ws + off);
     set_hull(a, ws, wl);
+    // One pass, no windows and room behind its dS: the parts of a split of
+    // every dK/dV block.
+    const size_t split = dkv_split_bytes(batch, heads_q, heads_kv, len_q, len_k, head_dim, key_mask != nullptr);
+    const size_t end = off + (size_t)a.nkv * per;
+    if (kv_per_pass == a.nkv && !window_lo && split > 0 && workspace_bytes >= end + split)
+      a.split_all = reinterpret_cast<float*>(ws + end);
   }
   return launch_status(launch_bwd(a, head_dim, kv_per_pass, s));
 }

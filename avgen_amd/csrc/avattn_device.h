@@ -257,6 +257,17 @@ __device__ __forceinline__ int xcd_remap(int bid, int total) {
   return xcd * per + (xcd < rem ? xcd : rem) + local;
 }
 
+// xcd_remap for calls with a key mask: whole (batch, kv head) pairs of `per`
+// blocks still stay on one XCD, but XCD x takes pairs x, x + 8, ..., so that a
+// batch row with few attended keys leaves no XCD idle.  Needs total = pairs *
+// per with pairs a multiple of 8, else the plain map.
+__device__ __forceinline__ int xcd_remap_pairs(int bid, int total, int per, bool masked) {
+  constexpr int kXcds = 8;
+  if (!masked || total / per % kXcds != 0 || total % per != 0) return xcd_remap(bid, total);
+  const int local = bid / kXcds;
+  return (bid % kXcds + kXcds * (local / per)) * per + local % per;
+}
+
 // An int of device memory the kernel only reads, loaded through the constant
 // address space: with a wave-uniform address this is a scalar load.  (The
 // kernels' inline-asm stores clobber "memory", so the compiler cannot prove

@@ -204,6 +204,9 @@ struct BwdArgs {
   // parts in order and writes dk and dv.
   float* split_part;
   int nsplit, nparts;
+  // Slots for a split of every block (null: none; see dkv_split_plan), in
+  // place of split_part.
+  float* split_all;
 };
 
 // Partial-sum slots of the dK/dV tail split, 256 x D floats each; the
@@ -239,6 +242,10 @@ inline TailSplit plan_tail_split(int64_t total, int cus, int max_slots) {
   }
   return t;
 }
+
+// Split of every block of a short dK/dV grid of `total` 128-key blocks, each
+// over `tiles` 64-row query tiles (attn_bwd.hip); {0, 0}: none.
+TailSplit dkv_split_plan(int64_t total, int tiles, int D, bool masked);
 
 // Bytes of staged dS per (b, kv head) pair: dense, or the compact layout's
 // units_per_head units per query head.

@@ -482,7 +482,7 @@ def _bwd_windowed_impl(dout, q, k, v, out, lse, window_lo, window_hi, key_mask, 
             _stream(q.device),
         )
     else:
-        ws = _alloc_bwd_workspace(B, Hq, Hkv, Lq, Lk, D, q.device, stage_ds=True)
+        ws = _alloc_bwd_workspace(B, Hq, Hkv, Lq, Lk, D, q.device, stage_ds=True, windows=True)
         st = lib.avattn_bwd_windowed(
             *common_head,
             float(scale),
@@ -648,19 +648,24 @@ def bwd_workspace_plan(B, Hq, Hkv, Lq, Lk, D, device, stage_ds=None):
     return lib.avattn_bwd_staged_workspace_size(B, Hq, Hkv, Lq, Lk, D, int(pairs)), True
 
 
-def _alloc_bwd_workspace(B, Hq, Hkv, Lq, Lk, D, device, stage_ds=None, ds_units=0) -> torch.Tensor:
+def _alloc_bwd_workspace(B, Hq, Hkv, Lq, Lk, D, device, stage_ds=None, ds_units=0,
+                         windows=False) -> torch.Tensor:
     """The workspace of :func:`bwd_workspace_plan`, allocated; if the caching
     allocator cannot provide it (memory held by activations, say), the
     staged pairs per pass halve until it can (more passes, the same
     results), and with staging optional (``stage_ds`` not True) a last
     attempt goes without staging (the recomputing dQ kernel).  ``ds_units``:
-    the compact layout of key windows (units per query head)."""
+    the compact layout of key windows (units per query head); ``windows``: key
+    windows in the dense layout.  All pairs in one pass without windows: also
+    room for a split dK/dV grid."""
     lib = _lib.load()
     pairs = _staged_pairs(B, Hq, Hkv, Lq, Lk, D, device, stage_ds, ds_units)
 
     def staged_size(p):
         if ds_units:
             return lib.avattn_bwd_compact_workspace_size(B, Hq, Hkv, Lq, Lk, D, int(p), int(ds_units))
+        if p == B * Hkv and not windows:  # one pass: room for a split dK/dV grid too
+            return lib.avattn_bwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D)
         return lib.avattn_bwd_staged_workspace_size(B, Hq, Hkv, Lq, Lk, D, int(p))
 
     while pairs > 0:

@@ -238,7 +238,7 @@ def _ring_backward_into(grad_out, query, key, value, out, lse, key_mask, cp, sca
     Hkv = key.shape[1]
     bounds = [shard_bounds(L, cp, r) for r in range(cp)]
     masks = [None if key_mask is None else key_mask[:, a:b] for a, b in bounds]
-    full = max(lib.avattn_bwd_staged_workspace_size(B, Hq, Hkv, Lq, b - a, D, B * Hkv) for a, b in bounds)
+    full = max(lib.avattn_bwd_split_workspace_size(B, Hq, Hkv, Lq, b - a, D) for a, b in bounds)
     if overlap and not (cp > 1 and full > 0):
         overlap = False
     if overlap:

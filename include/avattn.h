@@ -190,6 +190,17 @@ size_t avattn_bwd_staged_workspace_size(int32_t batch, int32_t heads_q, int32_t 
                                         int32_t kv_pairs_per_pass);
 
 /*
+ * Workspace with which avattn_bwd and avattn_ring_bwd_step (staging dS,
+ * every (batch, kv head) pair in one pass) also split the key blocks of a
+ * short dK/dV grid over ranges of queries where that is faster; dk and dv
+ * then differ from the unsplit ones in rounding only.  0 for a problem the
+ * backward would refuse or that is empty.
+ */
+size_t avattn_bwd_split_workspace_size(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t len_q, int32_t len_k,
+                                       int32_t head_dim);
+
+
+/*
  * Forward with q k^T on fp8 (OCP e4m3) operands: per-head scales
  * q_scale[heads_q], k_scale[heads_kv] (device float32, e.g. from
  * avattn_fp8_absmax_scales).  k8 = e4m3(k * (1/k_scale[hk])) (fp32 multiply
