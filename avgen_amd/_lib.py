@@ -38,6 +38,19 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
          c_ptr, c_size,
          c_ptr],
     ),
+    "avattn_fwd_rotary": (
+        ctypes.c_int,
+        [c_ptr, c_ptr, c_ptr, c_i64p, c_i64p, c_i64p,
+         c_i32, c_i32, c_i32, c_i32, c_i32, c_i32,
+         c_ptr, c_i64,
+         c_ptr, c_ptr, c_i64,
+         c_ptr, c_ptr, c_i64,
+         c_f32,
+         c_ptr, c_i64p,
+         c_ptr,
+         c_ptr, c_size,
+         c_ptr],
+    ),
     "avattn_fwd_noalloc": (
         ctypes.c_int,
         [c_ptr, c_ptr, c_ptr, c_i64p, c_i64p, c_i64p,

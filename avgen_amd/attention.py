@@ -264,8 +264,9 @@ def rotary_attention(
     query rotation fused into the kernel's Q load
     (src/avgen/models/layers.py:533-544).
 
-    The key is rotated once by the standalone rotary kernel (every query tile
-    re-reads K, so rotating per load would multiply its traffic).  The result
+    The key is rotated once (every query tile re-reads K, so rotating per load
+    would multiply its traffic): in the forward's padded copy of it, or by the
+    standalone rotary kernel where a backward may follow.  The result
     equals the unfused composition bit for bit.  ``key_tables`` defaults to
     ``tables`` (self-attention); pass the key shard's tables for a KV chunk.
     """
@@ -273,10 +274,9 @@ def rotary_attention(
         return torch.zeros_like(query)
     _validate(query, key, value, 0.0, False, enable_gqa)
     kt = tables if key_tables is None else key_tables
-    k_rot = ops.rope_apply(key, kt.cos, kt.sin, False)
     mask = _as_key_mask(attn_mask, query.shape[0], query.shape[-2], key.shape[-2])
-    out, _ = ops.flash_fwd(query, k_rot, value, mask, tables.cos, tables.sin, ops.default_scale(query.shape[-1]))
-    return out
+    return ops.rotary_fwd(query, key, value, mask, tables.cos, tables.sin, kt.cos, kt.sin,
+                          ops.default_scale(query.shape[-1]))
 
 
 def attention_fp8(

@@ -314,6 +314,25 @@ int avattn_fwd(const void* q, const void* k, const void* v, const int64_t* q_str
                   nullptr, scale, out, out_strides, lse, workspace, workspace_bytes, stream);
 }
 
+int avattn_fwd_rotary(const void* q, const void* k, const void* v, const int64_t* q_strides, const int64_t* k_strides,
+                      const int64_t* v_strides, int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t len_q,
+                      int32_t len_k, int32_t head_dim, const uint8_t* key_mask, int64_t key_mask_batch_stride,
+                      const float* rope_cos_q, const float* rope_sin_q, int64_t rope_q_batch_stride,
+                      const float* rope_cos_k, const float* rope_sin_k, int64_t rope_k_batch_stride, float scale,
+                      void* out, const int64_t* out_strides, float* lse, void* workspace, size_t workspace_bytes,
+                      avattn_stream_t stream) {
+  const int st = check_tables(rope_cos_k, rope_sin_k, rope_k_batch_stride);
+  if (st != AVATTN_OK) return st;
+  RingOpts keys;  // the key tables alone: no running merge
+  keys.cos_k = rope_cos_k;
+  keys.sin_k = rope_sin_k;
+  keys.rksb = rope_k_batch_stride;
+  return fwd_impl(q, k, v, q_strides, k_strides, v_strides, batch, heads_q, heads_kv, len_q, len_k, head_dim,
+                  key_mask, key_mask_batch_stride, rope_cos_q, rope_sin_q, rope_q_batch_stride, false, nullptr,
+                  nullptr, scale, out, out_strides, lse, workspace, workspace_bytes, stream, nullptr, nullptr, 0,
+                  &keys);
+}
+
 int avattn_fwd_fp8(const void* q, const void* k, const void* v, const int64_t* q_strides, const int64_t* k_strides,
                    const int64_t* v_strides, int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t len_q,
                    int32_t len_k, int32_t head_dim, const uint8_t* key_mask, int64_t key_mask_batch_stride,

@@ -139,6 +139,19 @@ def _direct(function, op, impl, args, tensors):
     return impl(*args)
 
 
+def rotary_fwd(q, k, v, key_mask, cos_q, sin_q, cos_k, sin_k, scale):
+    """Attention output of unrotated ``q`` and ``k``.  A plain bf16 call without
+    grad rotates k inside the forward's copy of it, where a launch and a pass
+    of its own took (2,20,3600,128) from 296 to 304 us; otherwise the rotation
+    is its own op, which the backward needs.  The same bits."""
+    tensors = (q, k, v, key_mask, cos_q, sin_q, cos_k, sin_k)
+    if (k.dtype is torch.bfloat16 and _plain_eager(*tensors)
+            and not (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors))):
+        _check_tables("avgen_amd.rope_apply", cos_k, sin_k, k.shape[0], k.shape[2], k.shape[3])
+        return _fwd_impl(q, k, v, key_mask, cos_q, sin_q, scale, key_tables=(cos_k, sin_k))[0]
+    return flash_fwd(q, rope_apply(k, cos_k, sin_k, False), v, key_mask, cos_q, sin_q, scale)[0]
+
+
 def _grad_direct(*tensors) -> bool:
     """Whether a backward formula may call an implementation instead of its
     op: plain eager and not itself differentiated (create_graph)."""
@@ -236,7 +249,9 @@ def _check_tables(name: str, cos: torch.Tensor, sin: torch.Tensor, batch: int, l
 # ---------------------------------------------------------------------------
 
 
-def _fwd_impl(q, k, v, key_mask, rope_cos, rope_sin, scale):
+def _fwd_impl(q, k, v, key_mask, rope_cos, rope_sin, scale, key_tables=None):
+    """``key_tables`` (bf16 only): ``(cos, sin)`` that rotate an unrotated ``k``
+    in its padded copy."""
     name = "avgen_amd.flash_fwd"
     _check_qkv(name, q, k, v, allow_f32=True)
     _require_gpu(name, q, k, v, key_mask, rope_cos, rope_sin)
@@ -256,11 +271,16 @@ def _fwd_impl(q, k, v, key_mask, rope_cos, rope_sin, scale):
     lse = torch.empty((B, Hq, Lq), device=q.device, dtype=torch.float32)
     lib = _lib.load()
     ws = _workspace(lib.avattn_fwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D, 0), q.device)
-    st = lib.avattn_fwd(
+    fwd, key_args = lib.avattn_fwd, ()
+    if key_tables is not None:
+        cos_k, sin_k, rksb = _check_tables(name, *key_tables, B, Lk, D)
+        fwd, key_args = lib.avattn_fwd_rotary, (_ptr(cos_k), _ptr(sin_k), rksb)
+    st = fwd(
         _ptr(q), _ptr(k), _ptr(v), _strides3(q), _strides3(k), _strides3(v),
         B, Hq, Hkv, Lq, Lk, D,
         _ptr(mask), msb,
         _ptr(rope_cos), _ptr(rope_sin), rsb,
+        *key_args,
         float(scale),
         _ptr(out), _strides3(out), _ptr(lse),
         _ptr(ws), ws.numel(),

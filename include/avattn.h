@@ -116,6 +116,28 @@ int avattn_fwd(const void* q, const void* k, const void* v,
                avattn_stream_t stream);
 
 /*
+ * avattn_fwd on unrotated keys: k is rotated with its own tables (element
+ * (b, 0, j, p) at b * rope_k_batch_stride + j * (head_dim/2) + p) as its
+ * padded copy is made.  The bits of avattn_rope_apply on k followed by
+ * avattn_fwd, without that pass over k (src/avgen/models/layers.py:533-544).
+ */
+int avattn_fwd_rotary(const void* q, const void* k, const void* v,
+                      const int64_t* q_strides, const int64_t* k_strides,
+                      const int64_t* v_strides,
+                      int32_t batch, int32_t heads_q, int32_t heads_kv,
+                      int32_t len_q, int32_t len_k, int32_t head_dim,
+                      const uint8_t* key_mask, int64_t key_mask_batch_stride,
+                      const float* rope_cos_q, const float* rope_sin_q,
+                      int64_t rope_q_batch_stride,
+                      const float* rope_cos_k, const float* rope_sin_k,
+                      int64_t rope_k_batch_stride,
+                      float scale,
+                      void* out, const int64_t* out_strides,
+                      float* lse,
+                      void* workspace, size_t workspace_bytes,
+                      avattn_stream_t stream);
+
+/*
  * avattn_fwd without a workspace argument and without any allocation: no
  * counterpart in the reference; for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
