@@ -342,32 +342,14 @@ __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(F32Args a) {
 template <int D>
 __global__ __launch_bounds__(64) void fwd_f32_combine_kernel(F32Args a) {
   constexpr int DT = D / 32, SLOT = fwd_slot_floats(32, D);
-  const int lane = threadIdx.x, l32 = lane & 31;
+  const int l32 = threadIdx.x & 31;
   const int sb = blockIdx.x / 4, wave = blockIdx.x % 4;
   const int nqb = (a.Lq + 127) / 128;
   const int bid = nqb * a.B * a.Hq - a.nsplit + sb;
   const float* slot = a.part + ((int64_t)sb * a.nparts * 4 + wave) * SLOT;
-  float m = kNegInf;
-  for (int p = 0; p < a.nparts; ++p) m = fmaxf(m, slot[(int64_t)p * 4 * SLOT + 32 * D + l32]);
   f32x16 o[DT];
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt) o[dt] = zero16();
-  float l = 0.f;
-  for (int p = 0; p < a.nparts; ++p) {
-    const float* sp = slot + (int64_t)p * 4 * SLOT;
-    const float mp = sp[32 * D + l32];
-    // no attended key in this part (mp -inf): nothing, unless a NaN reached it
-    const float w = mp == kNegInf ? 0.f : __builtin_amdgcn_exp2f((mp - m) * a.c);
-    l = fmaf(sp[32 * D + 32 + l32], w, l);
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 x = ld4(sp + ((dt * 4 + g) * 64 + lane) * 4);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[dt][4 * g + r] = fmaf(x[r], w, o[dt][4 * g + r]);
-      }
-  }
+  float m, l;
+  combine_parts<D>(slot, 4 * SLOT, a.nparts, a.c, o, m, l);
   const int row = bid % nqb * 128 + wave * 32 + l32;
   if (row < a.Lq) write_row_f32<D>(a, o, m, l, bid / nqb, row);
 }

@@ -846,37 +846,16 @@ template <int D, int BM>
 __global__ __launch_bounds__(256) void fwd_combine_kernel(FwdArgs a, float c, float unit) {
   constexpr int DT = D / 32;
   __shared__ __attribute__((aligned(16))) bf16 ep[4][32 * D];
-  const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int l32 = lane & 31;
   const int u = blockIdx.x * 4 + wave;  // 32-row group of the split blocks
   const int s = u / (BM / 32), w = u % (BM / 32);
   const int nqt = (a.Lq + BM - 1) / BM;
   const int bid = nqt * a.B * a.Hq - a.nsplit + s;
   const int row0 = bid % nqt * BM + w * 32;
   const float* slot = a.part + (int64_t)s * a.nparts * fwd_slot_floats(BM, D) + (int64_t)w * fwd_slot_floats(32, D);
-  float m = kNegInf;
-  for (int p = 0; p < a.nparts; ++p) m = fmaxf(m, slot[p * fwd_slot_floats(BM, D) + 32 * D + l32]);
-  float l = 0.f;
+  float m, l;
   f32x16 acc[DT];
-#pragma unroll
-  for (int i = 0; i < DT; ++i) acc[i] = zero16();
-  for (int p = 0; p < a.nparts; ++p) {
-    const float* sp = slot + p * fwd_slot_floats(BM, D);
-    const float mp = sp[32 * D + l32];
-    // a part without an attended key (mp -inf) weighs nothing, unless a NaN
-    // reached its sum or output
-    const float wt = mp == kNegInf ? 0.f : __builtin_amdgcn_exp2f((mp - m) * c);
-    l = fmaf(sp[32 * D + 32 + l32], wt, l);
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 x = *reinterpret_cast<const f32x4*>(sp + ((dt * 4 + g) * 64 + lane) * 4);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[dt][4 * g + r] = fmaf(x[r], wt, acc[dt][4 * g + r]);
-      }
-  }
+  combine_parts<D>(slot, fwd_slot_floats(BM, D), a.nparts, c, acc, m, l);
   float inv, lse;
   row_state(m, l, unit, inv, lse);
   write_rows<D>(a, acc, inv, lse, ep[wave], bid / nqt, row0);

@@ -268,6 +268,56 @@ __device__ __forceinline__ int xcd_remap_pairs(int bid, int total, int per, bool
   return (bid % kXcds + kXcds * (local / per)) * per + local % per;
 }
 
+// The parts of 32 split forward rows, each fwd_slot_floats(32, D) floats (the
+// accumulators in lane order, then the rows' maxima and sums) `stride` floats
+// apart, added in order, each scaled from its own maximum to the largest.
+// nparts is 2..8.  What bounds it is the latency of reads that other XCDs just
+// wrote (about 0.8 us each): the maxima and sums of all parts are read at once
+// and the accumulators of several parts together, so a row group waits for 3
+// (D 64) or 5 (D 128) of them where one part at a time took 16: float32
+// (1,4,1024,64) 8.9 -> 5.2 us, (2,20,3600,128) 10.1 -> 7.3.
+template <int D>
+__device__ __forceinline__ void combine_parts(const float* slot, int64_t stride, int nparts, float c,
+                                              f32x16 (&acc)[D / 32], float& m, float& l) {
+  constexpr int DT = D / 32, MAXP = 8, G = 256 / D;  // G parts of accumulators in flight
+  const int lane = threadIdx.x & 63, l32 = lane & 31;
+  float mp[MAXP], lp[MAXP];
+#pragma unroll
+  for (int p = 0; p < MAXP; ++p) {
+    const float* sp = slot + min(p, nparts - 1) * stride + 32 * D + l32;  // past the last part: it again
+    mp[p] = sp[0];
+    lp[p] = sp[32];
+  }
+  m = kNegInf;
+  l = 0.f;
+#pragma unroll
+  for (int p = 0; p < MAXP; ++p) m = fmaxf(m, mp[p]);
+#pragma unroll
+  for (int i = 0; i < DT; ++i) acc[i] = zero16();
+#pragma unroll
+  for (int p0 = 0; p0 < MAXP; p0 += G) {
+    if (p0 >= nparts) break;
+    f32x4 x[G][4 * DT];
+#pragma unroll
+    for (int p = 0; p < G; ++p)
+#pragma unroll
+      for (int j = 0; j < 4 * DT; ++j)
+        x[p][j] = *reinterpret_cast<const f32x4*>(slot + min(p0 + p, nparts - 1) * stride + (j * 64 + lane) * 4);
+#pragma unroll
+    for (int p = 0; p < G; ++p) {
+      if (p0 + p >= nparts) break;
+      // a part without an attended key (maximum -inf) weighs nothing, unless a
+      // NaN reached its sum or output
+      const float w = mp[p0 + p] == kNegInf ? 0.f : __builtin_amdgcn_exp2f((mp[p0 + p] - m) * c);
+      l = fmaf(lp[p0 + p], w, l);
+#pragma unroll
+      for (int j = 0; j < 4 * DT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[j / 4][4 * (j % 4) + r] = fmaf(x[p][j][r], w, acc[j / 4][4 * (j % 4) + r]);
+    }
+  }
+}
+
 // An int of device memory the kernel only reads, loaded through the constant
 // address space: with a wave-uniform address this is a scalar load.  (The
 // kernels' inline-asm stores clobber "memory", so the compiler cannot prove
