@@ -273,6 +273,13 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
          c_ptr, c_ptr, c_i64, c_i32,
          c_ptr, c_i64p, c_ptr],
     ),
+    "avattn_rope_apply_pair_f32": (
+        ctypes.c_int,
+        [c_i32, c_i32,
+         c_ptr, c_i64p, c_i32, c_i32, c_ptr, c_ptr, c_i64, c_ptr, c_i64p,
+         c_ptr, c_i64p, c_i32, c_i32, c_ptr, c_ptr, c_i64, c_ptr, c_i64p,
+         c_ptr],
+    ),
 }
 
 # Status codes (include/avattn.h).

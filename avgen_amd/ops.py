@@ -140,14 +140,17 @@ def _direct(function, op, impl, args, tensors):
 
 
 def rotary_fwd(q, k, v, key_mask, cos_q, sin_q, cos_k, sin_k, scale):
-    """Attention output of unrotated ``q`` and ``k``.  A plain bf16 call without
+    """Attention output of unrotated ``q`` and ``k``.  A plain float32 call without
+    grad rotates both in one launch (``_rotary_fwd_f32``).  A plain bf16 call without
     grad rotates k inside the forward's copy of it, where a launch and a pass
     of its own took (2,20,3600,128) from 296 to 304 us; otherwise the rotation
     is its own op, which the backward needs.  The same bits."""
     tensors = (q, k, v, key_mask, cos_q, sin_q, cos_k, sin_k)
-    if (k.dtype is torch.bfloat16 and _plain_eager(*tensors)
+    if (k.dtype in (torch.bfloat16, torch.float32) and _plain_eager(*tensors)
             and not (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors))):
-        _check_tables("avgen_amd.rope_apply", cos_k, sin_k, k.shape[0], k.shape[2], k.shape[3])
+        cos_k, sin_k, ks = _check_tables("avgen_amd.rope_apply", cos_k, sin_k, k.shape[0], k.shape[2], k.shape[3])
+        if k.dtype is torch.float32:
+            return _rotary_fwd_f32(q, k, v, key_mask, cos_q, sin_q, cos_k, sin_k, ks, scale)
         return _fwd_impl(q, k, v, key_mask, cos_q, sin_q, scale, key_tables=(cos_k, sin_k))[0]
     return flash_fwd(q, rope_apply(k, cos_k, sin_k, False), v, key_mask, cos_q, sin_q, scale)[0]
 
@@ -311,6 +314,24 @@ def _fwd_f32_impl(name, q, k, v, key_mask, rope_cos, rope_sin, scale):
     if rope_cos is not None:
         q = _rope_apply_impl(q, rope_cos, rope_sin, False)
     return _fwd_f32_launch(name, q, k, v, None, None, 0, key_mask, scale)
+
+
+def _rotary_fwd_f32(q, k, v, key_mask, cos_q, sin_q, cos_k, sin_k, k_table_stride, scale):
+    name = "avgen_amd.flash_fwd"
+    _check_qkv(name, q, k, v, allow_f32=True)
+    B, Hq, Lq, D = q.shape
+    cos_q, sin_q, q_table_stride = _check_tables("avgen_amd.rope_apply", cos_q, sin_q, B, Lq, D)
+    q, k = _f32_ready(q), _f32_ready(k)
+    qr = _f32_ready(torch.empty_like(q, memory_format=torch.preserve_format))
+    kr = _f32_ready(torch.empty_like(k, memory_format=torch.preserve_format))
+    st = _lib.load().avattn_rope_apply_pair_f32(
+        B, D,
+        _ptr(q), _strides3(q), Hq, Lq, _ptr(cos_q), _ptr(sin_q), q_table_stride, _ptr(qr), _strides3(qr),
+        _ptr(k), _strides3(k), k.shape[1], k.shape[2], _ptr(cos_k), _ptr(sin_k), k_table_stride, _ptr(kr), _strides3(kr),
+        _stream(q.device),
+    )
+    _lib.check(st, "avgen_amd.rope_apply")
+    return _fwd_f32_launch(name, qr, kr, v, None, None, 0, key_mask, scale)[0]
 
 
 def _fwd_f32_launch(name, q, k, v, lo, hi, wsb, key_mask, scale):

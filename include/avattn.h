@@ -841,6 +841,16 @@ int avattn_rope_apply_f32(const float* x, const int64_t* x_strides,
                           float* out, const int64_t* out_strides,
                           avattn_stream_t stream);
 
+/* avattn_rope_apply_f32 (not inverse) on a query and a key, one launch. */
+int avattn_rope_apply_pair_f32(int32_t batch, int32_t head_dim,
+                               const float* q, const int64_t* q_strides, int32_t heads_q, int32_t len_q,
+                               const float* cos_q, const float* sin_q, int64_t table_q_batch_stride,
+                               float* q_out, const int64_t* q_out_strides,
+                               const float* k, const int64_t* k_strides, int32_t heads_k, int32_t len_k,
+                               const float* cos_k, const float* sin_k, int64_t table_k_batch_stride,
+                               float* k_out, const int64_t* k_out_strides,
+                               avattn_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

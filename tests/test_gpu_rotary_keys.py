@@ -52,6 +52,23 @@ def test_same_bits_as_rotating_k_first(B, H, Hkv, Lq, Lk, D, tb, layout, masked)
     assert grad.requires_grad and torch.equal(grad.detach(), ref)
 
 
+@pytest.mark.parametrize("layout", ["bhld", "blhd", "shared", "offset"])
+@pytest.mark.parametrize("B,H,Hkv,Lq,Lk,D,tb", [(1, 1, 1, 1, 2, 64, 1), (2, 4, 2, 63, 165, 64, 2),
+                                                (1, 3, 1, 257, 31, 128, 1)])
+def test_float32_pair_has_the_bits_of_two_rotations(B, H, Hkv, Lq, Lk, D, tb, layout):
+    from avgen_amd import attention as A
+    from avgen_amd import ops
+
+    q, k, v, tq, tk = _case(B, H, Hkv, Lq, Lk, D, layout, tb)
+    q, k, v = q.float(), k.float(), v.float()
+    mask = torch.arange(Lk, device="cuda")[None] < max(1, Lk // 2)
+    with torch.no_grad():
+        out = A.rotary_attention(q, k, v, tq, key_tables=tk, enable_gqa=True, attn_mask=mask[:, None, None, :])
+        qr, kr = ops.rope_apply(q, tq.cos, tq.sin, False), ops.rope_apply(k, tk.cos, tk.sin, False)
+        ref, _ = ops.flash_fwd(qr, kr, v, mask, None, None, ops.default_scale(D))
+    assert torch.equal(out, ref)
+
+
 def test_errors_are_those_of_the_composition():
     from avgen_amd import attention as A
     from avgen_amd.rope import RotaryTables
@@ -64,6 +81,10 @@ def test_errors_are_those_of_the_composition():
             A.rotary_attention(q, k, v, tq, key_tables=RotaryTables(tk.cos.double(), tk.sin.double()))
         with pytest.raises(TypeError):
             A.rotary_attention(q.float(), k, v, tq, key_tables=tk)
+        with pytest.raises(TypeError):
+            A.rotary_attention(q, k.float(), v.float(), tq, key_tables=tk)
+        with pytest.raises(ValueError, match="rope_apply: sequence length 64 does not match"):
+            A.rotary_attention(q.float(), k.float(), v.float(), tk, key_tables=tk)
 
 
 def test_key_tables_are_checked_at_the_c_entry():
