@@ -295,11 +295,12 @@ __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(F32Args a) {
         for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
       m = mn;
     }
-    const float mc = m * a.c;
+    // No key yet: every score is -inf (p = 0) or NaN, which must reach the sum.
+    const float mc = m == kNegInf ? 0.f : m * a.c;
     f32x16 p;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      p[i] = m == kNegInf ? 0.f : __builtin_amdgcn_exp2f(fmaf(s[i], a.c, -mc));
+      p[i] = __builtin_amdgcn_exp2f(fmaf(s[i], a.c, -mc));
       l += p[i];
     }
     // O^T += V^T P^T: k-step j takes key 8*(j/4) + 4*hh + j%4, this lane's
