@@ -160,8 +160,10 @@ __device__ __forceinline__ void write_row_f32(const F32Args& a, const f32x16 (&o
 // the probabilities stay at most 2^8 and out = O / l is unchanged in exact
 // arithmetic.  WIN: per-row key windows (F32Args::wlo/whi): the workgroup
 // visits the tiles meeting its rows' windows and masks each score outside
-// its row's window.
-template <int D, bool WIN>
+// its row's window.  SPLIT: the grid has split row blocks (F32Args::nsplit);
+// without them the same code ran 0.7-1% slower ((2,20,8192,128) 10.35 against
+// 10.44 ms, (1,16,6000,64) 1,213 against 1,233 us).
+template <int D, bool WIN, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(F32Args a) {
   constexpr int KT = 32, ROWS = 128, PITCH = D + 4, HD = D / 2, DT = D / 32;
   constexpr int PER = KT * D / 4 / 256;  // K float4 chunks per thread and tile
@@ -174,8 +176,8 @@ __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(F32Args a) {
   const int l32 = lane & 31, hh = lane >> 5;
   const int nqb = (a.Lq + ROWS - 1) / ROWS;
   const int total = nqb * a.B * a.Hq;
-  int bid, part;
-  split_block(a, total, bid, part);
+  int bid = blockIdx.x, part = -1;
+  if constexpr (SPLIT) split_block(a, total, bid, part);
   const int qb = bid % nqb, bh = bid / nqb;
   const int b = bh / a.Hq, h = bh % a.Hq, hk = h / (a.Hq / a.Hkv);
   const int row = qb * ROWS + wave * 32 + l32;
@@ -241,7 +243,7 @@ __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(F32Args a) {
     if (valid) row_window(a, b, row, wl, wh);
     window_tiles<4>(wl, wh, valid, red, t0, ntile);
   }
-  if (part >= 0) {  // this part's share of the tiles (possibly none)
+  if (SPLIT && part >= 0) {  // this part's share of the tiles (possibly none)
     const int n = ntile - t0;
     ntile = t0 + n * (part + 1) / a.nparts;
     t0 += n * part / a.nparts;
@@ -322,7 +324,7 @@ __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(F32Args a) {
   }
 
   l = halves_sum(l);
-  if (part >= 0) {
+  if (SPLIT && part >= 0) {
     // One part of split rows: raw accumulators, maximum and sum, in the lane
     // order fwd_f32_combine_kernel reads them in.
     float* slot = a.part + (((int64_t)(bid - total + a.nsplit) * a.nparts + part) * 4 + wave) * fwd_slot_floats(32, D);
@@ -809,18 +811,17 @@ __global__ __launch_bounds__(512) void bwd_dq_f32_kernel(F32Args a) {
   }
 }
 
-// dQ = scale * dS K from the staged dS: four waves per workgroup, 32 query
-// rows each (two or more workgroups per CU fill a short last round better
-// than one of eight waves did), 32-key tiles of K in LDS (the backward tile layout).  A lane
+// dQ = scale * dS K from the staged dS: NW (4 or 8) waves per workgroup, 32
+// query rows each, 32-key tiles of K in LDS (the backward tile layout).  A lane
 // reads its row's dS over keys 16*(l/32) .. +15 of a tile (64 contiguous
 // bytes of the tile's 32x32 block) straight into registers, a tile ahead;
 // k-step j contracts keys j and 16 + j, so one LDS read gives the lane its
 // D/32 channel blocks of K's row 16*(l/32) + j.  WIN: the workgroup stages
 // the tiles meeting its rows' windows, and a wave multiplies only the key
 // blocks its rows meet (the blocks the windowed dK/dV kernel wrote).
-template <int D, bool WIN>
-__global__ __launch_bounds__(256, 2) void bwd_dq_ds_f32_kernel(F32Args a) {
-  constexpr int KT = 32, ROWS = 128, PITCH = D + 4, DT = D / 32;
+template <int D, bool WIN, int NW>
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void bwd_dq_ds_f32_kernel(F32Args a) {
+  constexpr int KT = 32, ROWS = 32 * NW, PITCH = D + 4, DT = D / 32;
   using vdt = float __attribute__((ext_vector_type(DT)));
   __shared__ __attribute__((aligned(16))) float ks[2][KT * PITCH];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -836,9 +837,9 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_ds_f32_kernel(F32Args a) {
   const bool valid = r0 + l32 < a.Lq;
   int wl = 0, wh = a.Lk, t0 = 0, ntile_w = ntile;
   if constexpr (WIN) {
-    __shared__ int red[8];
+    __shared__ int red[2 * NW];
     if (valid) row_window(a, b, r0 + l32, wl, wh);
-    window_tiles<4>(wl, wh, valid, red, t0, ntile_w);
+    window_tiles<NW>(wl, wh, valid, red, t0, ntile_w);
   }
   // does this wave multiply key tile t
   auto takes = [&](int t) {
@@ -851,7 +852,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_ds_f32_kernel(F32Args a) {
 #pragma unroll
   for (int d = 0; d < DT; ++d) dq[d] = zero16();
   const float* kb = a.k + b * a.ksb + hk * a.ksh;
-  Tile32<D, 256> sk;
+  Tile32<D, 64 * NW> sk;
   f32x4 pa[4];
   auto fetch = [&](int t) {
     sk.fetch(kb, a.ksl, t * KT, a.Lk, tid);
@@ -1175,8 +1176,12 @@ template <int D, bool WIN>
 void launch_fwd_f32(const F32Args& a, hipStream_t s) {
   const int64_t blocks = (int64_t)((a.Lq + 127) / 128) * a.B * a.Hq;
   const dim3 grid((unsigned)(blocks - a.nsplit + (int64_t)a.nsplit * a.nparts));
-  hipLaunchKernelGGL((fwd_f32_kernel<D, WIN>), grid, dim3(256), 0, s, a);
-  if (a.nsplit > 0) hipLaunchKernelGGL(fwd_f32_combine_kernel<D>, dim3(4 * a.nsplit), dim3(64), 0, s, a);
+  if (a.nsplit == 0) {
+    hipLaunchKernelGGL((fwd_f32_kernel<D, WIN, false>), grid, dim3(256), 0, s, a);
+    return;
+  }
+  hipLaunchKernelGGL((fwd_f32_kernel<D, WIN, true>), grid, dim3(256), 0, s, a);
+  hipLaunchKernelGGL(fwd_f32_combine_kernel<D>, dim3(4 * a.nsplit), dim3(64), 0, s, a);
 }
 
 // Staged dS floats per (batch, kv head) pair (see F32Args::ds).
@@ -1192,6 +1197,24 @@ constexpr int dkv_f32_slot_floats(int D) { return 2 * 128 * D; }
 FwdSplit dkv_f32_split_plan(int64_t blocks, int D) {
   const TailSplit t = plan_tail_split(blocks, 256, kSplitSlots);
   return FwdSplit{t.nsplit, t.nparts, (size_t)t.nsplit * t.nparts * dkv_f32_slot_floats(D) * sizeof(float)};
+}
+
+// dQ from staged dS over `heads` query heads, in workgroups of 256 rows, or of
+// 128 (two per CU, which fill a partial last round better) where their rounds
+// are fewer by more than staging K twice as often costs them: measured 12%
+// per row at head_dim 128, 9% at 64.  Backward with 8 against 4 waves, D 128:
+// (1,20,4096) 1.25 rounds 3,714 against 3,570 us, (1,10,16384) 2.5 rounds
+// 26.94 against 26.51 ms; (1,28,4096) 1.75 rounds 4,754 against 4,914 us,
+// (2,20,8192) 5 rounds 26.08 against 26.69 ms.
+template <int D, bool WIN>
+void launch_dq_ds_f32(const F32Args& a, int heads, hipStream_t s) {
+  constexpr int kCus = 256;
+  constexpr float kRowCost = D == 64 ? 1.09f : 1.12f;
+  const int64_t n8 = (int64_t)((a.Lq + 255) / 256) * heads, n4 = (int64_t)((a.Lq + 127) / 128) * heads;
+  if (0.5f * kRowCost * ((n4 + kCus - 1) / kCus) < (n8 + kCus - 1) / kCus)
+    hipLaunchKernelGGL((bwd_dq_ds_f32_kernel<D, WIN, 4>), dim3((unsigned)n4), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((bwd_dq_ds_f32_kernel<D, WIN, 8>), dim3((unsigned)n8), dim3(512), 0, s, a);
 }
 
 // pairs_per_pass 0: dQ recomputes S and dP; else dS is staged for that many
@@ -1211,7 +1234,7 @@ void launch_bwd_f32(F32Args a, int pairs_per_pass, hipStream_t s) {
     hipLaunchKernelGGL((bwd_dq_f32_kernel<D, WIN>), dim3((unsigned)(nqb * a.B * a.Hq)), dim3(512), 0, s, a);
     return;
   }
-  const int group = a.Hq / a.Hkv, nrb = (a.Lq + 127) / 128;
+  const int group = a.Hq / a.Hkv;
   for (int p0 = 0; p0 < pairs; p0 += pairs_per_pass) {
     const int np = pairs - p0 < pairs_per_pass ? pairs - p0 : pairs_per_pass;
     a.pair0 = p0;
@@ -1223,7 +1246,7 @@ void launch_bwd_f32(F32Args a, int pairs_per_pass, hipStream_t s) {
     if (a.nsplit > 0)
       hipLaunchKernelGGL(dkv_f32_reduce_kernel<D>, dim3((unsigned)(a.nsplit * (2 * 128 * (D / 4) / 256))), dim3(256), 0,
                          s, a);
-    hipLaunchKernelGGL((bwd_dq_ds_f32_kernel<D, WIN>), dim3((unsigned)(nrb * np * group)), dim3(256), 0, s, a);
+    launch_dq_ds_f32<D, WIN>(a, np * group, s);
   }
 }
 

@@ -140,12 +140,13 @@ def test_backward_split_equals_unsplit(Hq, Hkv, Lq, Lk, D, variant):
 
 
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("Lq", [1, 31, 33, 127, 128, 129, 257])
-def test_dq_rows(Lq, D):
+@pytest.mark.parametrize("H,Lq", [(4, 1), (4, 31), (4, 33), (4, 127), (4, 128), (4, 129), (4, 257),
+                                  (200, 129), (200, 256), (100, 257), (66, 515)])  # 256-row workgroups
+def test_dq_rows(H, Lq, D):
     from avgen_amd import ops
 
-    q, do = _rnd(1, 4, Lq, D, seed=1), _rnd(1, 4, Lq, D, seed=2)
-    k, v = _rnd(1, 2, 75, D, seed=3), _rnd(1, 2, 75, D, seed=4)
+    q, do = _rnd(1, H, Lq, D, seed=1), _rnd(1, H, Lq, D, seed=2)
+    k, v = _rnd(1, H // 2, 75, D, seed=3), _rnd(1, H // 2, 75, D, seed=4)
     s = 1 / math.sqrt(D)
     out, lse = ops.flash_fwd(q, k, v, None, None, None, s)
     dq = ops.flash_bwd(do, q, k, v, out, lse, None, s)[0]
@@ -154,3 +155,6 @@ def test_dq_rows(Lq, D):
     dp = do.double() @ vd.transpose(-1, -2)
     ref = (p * (dp - (p * dp).sum(-1, keepdim=True)) * s) @ kd
     assert (dq - ref).abs().max() <= 1e-5 * ref.abs().max() + 1e-6
+    lo, hi = torch.zeros(Lq, dtype=torch.int32, device="cuda"), torch.full((Lq,), 75, dtype=torch.int32, device="cuda")
+    windowed = ops.flash_bwd_windowed(do, q, k, v, out, lse, lo, hi, None, s, monotone=True)[0]
+    assert torch.equal(windowed, dq)
