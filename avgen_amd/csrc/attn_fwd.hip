@@ -888,12 +888,20 @@ __global__ void attn_empty_kernel(bf16* o, int64_t osb, int64_t osh, int64_t osl
 //   D 128, few keys, where the prologue and output are a large part: SMALL
 //     (75,600 x 128 keys 521 -> 470 us, 20,000 x 256 74.7 -> 66.2, x 512
 //     within noise);
-//   D 128, at most one workgroup of 256 rows per CU: SMALL, which spreads
-//     over more CUs ((1,4,4096) 80.1 -> 75.5 us, (1,8,3000) 66.3 -> 62.6,
-//     (1,20,1024) 34.3 -> 32.0).
-constexpr int kSmallKeys = 512, kCus = 256;
+//   D 128, at most one workgroup of 128 rows per CU and up to 1,024 keys:
+//     SMALL, which spreads over more CUs ((1,8,1024) x 700 keys 25.4 -> 22.6
+//     us, (1,64,511) 33.0 -> 30.1, (1,200,128) 46.0 -> 41.7).  With more
+//     workgroups, CUs hold two of them and gain nothing on one of 256 rows
+//     ((1,24,2013) x 10,752 keys 271 us in 192 workgroups of 256 rows, 314 in
+//     384 of 128; (1,17,2048) x 1,500 44 against 54); with more keys, the
+//     two LDS stages hide less of the loads' latency than four do ((1,200,128)
+//     x 2,000 keys 120 against 129, (1,100,256) x 5,000 178 against 198) and
+//     splitting 256-row workgroups gains more ((1,12,2560) x 6,169 106 against
+//     117 us).
+constexpr int kSmallKeys = 512, kSmallRoundKeys = 1024, kCus = 256;
 static bool use_small(int B, int Hq, int Lq, int Lk, int head_dim) {
-  return head_dim == 64 || Lk <= kSmallKeys || (int64_t)((Lq + 255) / 256) * B * Hq <= kCus;
+  return head_dim == 64 || Lk <= kSmallKeys ||
+         (Lk <= kSmallRoundKeys && (int64_t)((Lq + 127) / 128) * B * Hq <= kCus);
 }
 
 // Split of the last round's row blocks over ranges of key tiles: the number
@@ -901,6 +909,10 @@ static bool use_small(int B, int Hq, int Lq, int Lk, int head_dim) {
 // it saves 4 us or more.  Times per tile and round and per workgroup as
 // measured on an MI355X; (1,4,4096,128) 78.7 -> 61.1 us, D 64 56.7 -> 41.0,
 // (1,16,4725,128) x 18,900 keys 844 -> 666, (1,8,18900,128) 1330 -> 1190.
+// An only round of 256-row workgroups on more than half the CUs stays whole:
+// it clocks higher than the estimate has it, and the splits it picks took
+// (1,20,1792,128) x 10,752 keys from 221 to 234 us, (1,24,1537) 245 to 253
+// (20,000 keys 0.94-1.02 of the whole).
 FwdSplit fwd_split_plan(int B, int Hq, int Lq, int Lk, int D, bool fp8, bool windows) {
   FwdSplit best{0, 0, 0};
   if (windows) return best;  // the tiles of a row block are known on the device only
@@ -926,6 +938,7 @@ FwdSplit fwd_split_plan(int B, int Hq, int Lq, int Lk, int D, bool fp8, bool win
   // The parts cost their partial sums, written and read at 4 TB/s, and the
   // combining launch.
   const float slot_bytes = 4.f * fwd_slot_floats(bm, D);
+  if (!small && r == (int64_t)((Lq + bm - 1) / bm) * B * Hq && r > kCus / 2) return best;
   float cost = rounds(r) * (ntile * tile_us + fixed_us) - 4.f;
   for (int p = 2; p <= 8 && ntile / p >= 8; ++p) {
     const float c = rounds(r * p) * (ntile * tile_us / p + fixed_us) + 5.f + r * p * slot_bytes * 0.5e-6f;

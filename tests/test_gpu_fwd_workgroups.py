@@ -15,8 +15,12 @@ pytestmark = pytest.mark.gpu
     (300, 1, 513, 128),      # 300 workgroups of 256 rows, one row each
     (52, 1281, 577, 128),    # six per head, the last of one row; last key tile of one
     (52, 1281, 512, 128),    # few keys: 128 rows
-    (256, 256, 640, 128),    # at most one workgroup per CU: 128 rows
+    (256, 256, 640, 128),    # one workgroup of 256 rows per CU
     (257, 256, 640, 128),
+    (128, 255, 640, 128),    # at most one workgroup of 128 rows per CU: 128 rows
+    (129, 255, 640, 128),
+    (4, 300, 1024, 128),     # ... and up to 1,024 keys
+    (4, 300, 1025, 128),
     (3, 129, 1, 128),
     (40, 385, 130, 64),
 ])
