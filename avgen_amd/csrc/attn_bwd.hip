@@ -1350,32 +1350,30 @@ static int cu_count() {
 }
 
 // Split of every key block of a short dK/dV grid (no windows) over 2..8 ranges
-// of query tiles (at least 8 each), or {0, 0}: for grids of at most one round,
-// and with a key mask of at most two, where blocks without an attended key
-// end at once and leave the rest unevenly spread (weighed as half of them).
-// Estimated from the time per 64-row tile and per workgroup and the parts'
-// traffic at 4 TB/s; a partial round clocks higher (see fwd_split_plan).
+// of query tiles (at least 8 each), or {0, 0}: for grids of at most one round
+// (beyond it the tail split shares out the last round).  Estimated from the
+// time per 64-row tile and per workgroup and the parts' traffic at 4 TB/s; a
+// partial round clocks higher (see fwd_split_plan).  A key mask changes
+// nothing: how many blocks it leaves without an attended key is known on the
+// device only, and a plan that counted on half of them made fully attended
+// calls slower ((1,5,12000,128) x 6,656 keys, 260 blocks, 552 us unsplit,
+// 623 split; (2,20,40000) x 1,024 with one row empty 1,511 against 1,612).
 // Backward: (1,16,20000,128) x 256 keys 498 -> 198 us, (1,20,10000) x 128 keys
-// 255 -> 104, (1,4,4096) self-attention 171 -> 150, 75,600 x 512 keys with
-// 388 and 0 attended (2 x 40 heads) 3.68 -> 2.86 ms; with 512 and 500
-// attended 5.28 -> 5.38.
-TailSplit dkv_split_plan(int64_t total, int tiles, int D, bool masked) {
+// 255 -> 104, (1,4,4096) self-attention 171 -> 150.
+TailSplit dkv_split_plan(int64_t total, int tiles, int D) {
   constexpr int kCus = 256;
   TailSplit best{0, 0};
-  if (total > (masked ? 2 * kCus : kCus)) return best;
+  if (total > kCus) return best;
   const float work_us = tiles * (D == 64 ? 1.1f : 1.9f), fixed_us = 8.f;
-  auto rounds = [&](int64_t n) {
-    const int rem = (int)(n % kCus);
-    return n / kCus + (rem == 0 ? 0.f : 1.f - 0.38f * (1.f - (float)rem / kCus));
+  auto cost = [&](int p) {
+    const int n = (int)total * p, rem = n % kCus;
+    const float rounds = n / kCus + (rem == 0 ? 0.f : 1.f - 0.38f * (1.f - (float)rem / kCus));
+    return rounds * (work_us / p + fixed_us) + (p > 1 ? 5.f + n * (1024.f * D) * 0.5e-6f : 0.f);
   };
-  auto cost = [&](int64_t n, int p) {
-    return rounds(n * p) * (work_us / p + fixed_us) + (p > 1 ? 5.f + n * p * (1024.f * D) * 0.5e-6f : 0.f);
-  };
-  auto mean = [&](int p) { return masked ? 0.5f * (cost(total, p) + cost((total + 1) / 2, p)) : cost(total, p); };
-  float c = mean(1) - 4.f;
+  float c = cost(1) - 4.f;
   for (int p = 2; p <= 8 && tiles / p >= 8; ++p) {
-    if (mean(p) < c) {
-      c = mean(p);
+    if (cost(p) < c) {
+      c = cost(p);
       best = TailSplit{(int)total, p};
     }
   }
@@ -1448,7 +1446,7 @@ static hipError_t launch_bwd_d(const BwdArgs& args, int kv_per_pass, hipStream_t
     TailSplit ts = p.split_part ? plan_tail_split(total, cus, kSplitSlots) : TailSplit{0, 0};
     if (p.split_all != nullptr) {
       // Every block split (the region holds the plan's parts).
-      ts = dkv_split_plan(total, (a.Lqp / 64) * (a.Hq / a.Hkv), D, mask);
+      ts = dkv_split_plan(total, (a.Lqp / 64) * (a.Hq / a.Hkv), D);
       p.split_part = p.split_all;
     }
     p.nsplit = ts.nsplit;

@@ -409,9 +409,9 @@ size_t avattn_bwd_staged_workspace_size(int32_t batch, int32_t heads_q, int32_t 
 
 namespace {
 // Bytes of the parts of a dK/dV grid with every block split (0: not split).
-size_t dkv_split_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lq, int32_t Lk, int32_t D, bool masked) {
+size_t dkv_split_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lq, int32_t Lk, int32_t D) {
   const TailSplit t = dkv_split_plan((int64_t)B * Hkv * ((Lk + 127) / 128),
-                                     (int)(transpose_padded_len(Lq) / 64 * (Hq / Hkv)), D, masked);
+                                     (int)(transpose_padded_len(Lq) / 64 * (Hq / Hkv)), D);
   return (size_t)t.nsplit * t.nparts * 256 * D * sizeof(float);
 }
 }  // namespace
@@ -420,10 +420,8 @@ size_t avattn_bwd_split_workspace_size(int32_t batch, int32_t heads_q, int32_t h
                                        int32_t head_dim) {
   if (check_bwd_dims(batch, heads_q, heads_kv, len_q, len_k, head_dim) != AVATTN_OK) return 0;
   if ((int64_t)batch * heads_q * len_q == 0 || len_k == 0) return 0;
-  const size_t plain = dkv_split_bytes(batch, heads_q, heads_kv, len_q, len_k, head_dim, false);
-  const size_t masked = dkv_split_bytes(batch, heads_q, heads_kv, len_q, len_k, head_dim, true);
   return avattn_bwd_staged_workspace_size(batch, heads_q, heads_kv, len_q, len_k, head_dim, batch * heads_kv) +
-         (plain > masked ? plain : masked);
+         dkv_split_bytes(batch, heads_q, heads_kv, len_q, len_k, head_dim);
 }
 
 // Compact staged-dS layout of a windowed backward (BwdArgs::ds_tab).
@@ -586,7 +584,7 @@ static int bwd_impl(const void* dout, const void* q, const void* k, const void* 
     set_hull(a, ws, wl);
     // One pass, no windows and room behind its dS: the parts of a split of
     // every dK/dV block.
-    const size_t split = dkv_split_bytes(batch, heads_q, heads_kv, len_q, len_k, head_dim, key_mask != nullptr);
+    const size_t split = dkv_split_bytes(batch, heads_q, heads_kv, len_q, len_k, head_dim);
     const size_t end = off + (size_t)a.nkv * per;
     if (kv_per_pass == a.nkv && !window_lo && split > 0 && workspace_bytes >= end + split)
       a.split_all = reinterpret_cast<float*>(ws + end);

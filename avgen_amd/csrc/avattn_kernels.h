@@ -245,7 +245,7 @@ inline TailSplit plan_tail_split(int64_t total, int cus, int max_slots) {
 
 // Split of every block of a short dK/dV grid of `total` 128-key blocks, each
 // over `tiles` 64-row query tiles (attn_bwd.hip); {0, 0}: none.
-TailSplit dkv_split_plan(int64_t total, int tiles, int D, bool masked);
+TailSplit dkv_split_plan(int64_t total, int tiles, int D);
 
 // Bytes of staged dS per (b, kv head) pair: dense, or the compact layout's
 // units_per_head units per query head.

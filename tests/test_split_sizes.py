@@ -27,3 +27,16 @@ def lib():
 def test_forward(lib, H, Lq, Lk, D, split, fp8):
     base = (lib.avattn_fwd_fp8_workspace_size if fp8 else lib.avattn_fwd_workspace_size)(1, H, Lk, D)
     assert (lib.avattn_fwd_split_workspace_size(1, H, H, Lq, Lk, D, fp8) > base) == split
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,Lq,Lk,split", [
+    (1, 16, 20000, 256, True),    # 32 key blocks
+    (2, 20, 20000, 256, True),    # 80
+    (1, 5, 12000, 6400, False),   # 250: nearly every CU
+    (1, 5, 12000, 6656, False),   # 260: more than one round
+    (2, 40, 75600, 512, False),
+])
+def test_backward(lib, B, H, Lq, Lk, D, split):
+    staged = lib.avattn_bwd_staged_workspace_size(B, H, H, Lq, Lk, D, B * H)
+    assert (lib.avattn_bwd_split_workspace_size(B, H, H, Lq, Lk, D) > staged) == split
