@@ -319,7 +319,10 @@ hipError_t launch_prep_fwd(const FwdArgs& a, int head_dim, hipStream_t stream) {
 hipError_t launch_prep_bwd(const BwdArgs& a, int head_dim, hipStream_t stream) {
   const int64_t nk = (int64_t)a.B * a.Hkv * (a.Lkp / 64);
   const int64_t qtiles = (int64_t)a.B * a.Hq * (a.Lqp / 64);
-  const int64_t nq = !a.reuse_q && a.qt == a.qr ? qtiles : 0, nd = !a.reuse_q && a.dt == a.dor ? qtiles : 0;
+  // Kept from an earlier call (reuse_q): the statistics and a rotated q copy.
+  // Copies that rows that overlap need are made again: that call may have read
+  // the same values in place, from rows that do not.
+  const int64_t nq = a.qt == a.qr && !(a.reuse_q && a.cos_q) ? qtiles : 0, nd = a.dt == a.dor ? qtiles : 0;
   const int rpb = 256 / (head_dim / 8) * kStatRows;
   const int64_t ns = a.reuse_q ? 0 : (int64_t)a.B * a.Hq * ((a.Lqp + rpb - 1) / rpb);
   if (nk + nq + nd + ns > 2147483647) return hipErrorInvalidValue;

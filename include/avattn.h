@@ -187,8 +187,9 @@ size_t avattn_fwd_split_workspace_size(int32_t batch, int32_t heads_q, int32_t h
 
 /*
  * Workspace bytes avattn_bwd needs for these sizes: two floats per query row
- * (softmax statistics), row-major copies of q and dout,
- * row-major copies of k and v and a head_dim-major copy of k (sequences
+ * (softmax statistics), room for row-major copies of q and dout (written
+ * only where avattn_bwd cannot read them in place) and of k and v (written
+ * without staged dS), and a head_dim-major copy of k (sequences
  * padded to multiples of 64), plus the padded per-key bias and per-32-key
  * flags, plus, when batch * heads_kv * ceil(len_k / 128) (dK/dV
  * workgroups) exceeds 256, 512 * 256 * head_dim floats of partial sums for
@@ -276,15 +277,19 @@ int avattn_fp8_absmax_scales(const void* x, const int64_t* x_strides,
  * chunk's contributions.  dk/dv of a masked key are exactly 0.  With
  * heads_kv < heads_q, dk/dv sum over the query heads of each group.
  * workspace must hold avattn_bwd_workspace_size() bytes; its query-side part
- * (statistics and the q/dout copies, at offsets that depend only on batch,
+ * (statistics and any q/dout copies, at offsets that depend only on batch,
  * heads_q, len_q and head_dim) may be kept between calls, everything else is
- * scratch for this call.
+ * scratch for this call.  q and dout are read in place unless their rows
+ * overlap (seq stride below head_dim) or lie 2^23 elements apart or more (or,
+ * in avattn_ring_bwd_step, q is rotated first); only then are they copied.
  * flags (bitwise or, 0 = neither):
  *   AVATTN_BWD_REUSE_QUERY_SIDE  the workspace already holds the query-side
  *       preparation of a previous avattn_bwd call with the same dout, q, out,
  *       lse, scale, batch, heads_q, len_q and head_dim (e.g. the previous KV
  *       chunk of one ring step); it is not recomputed.  The caller asserts
- *       this; stale contents give wrong gradients.
+ *       this; stale contents give wrong gradients.  dout and q are passed
+ *       again with the same values (they may be read in place), in any
+ *       layout.
  *   AVATTN_BWD_DQ_ACCUMULATE_F32 dq is float32 (strides in float elements,
  *       multiples of 4, 16-byte aligned) and this chunk's dq is added to it
  *       in fp32 (before any rounding) instead of being written as bf16: the
