@@ -167,6 +167,18 @@ def _workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     return torch.empty(max(int(nbytes), 256), device=device, dtype=torch.uint8)
 
 
+def _split_workspace(nbytes: int, base, device: torch.device) -> torch.Tensor:
+    """A workspace of ``nbytes``, with room for a split grid, or of ``base()``
+    bytes (the same call unsplit) where the allocator cannot provide that."""
+    try:
+        return _workspace(nbytes, device)
+    except torch.OutOfMemoryError:
+        smaller = base()
+        if smaller >= nbytes:
+            raise
+        return _workspace(smaller, device)
+
+
 def _require_gpu(name: str, *tensors: Optional[torch.Tensor]) -> None:
     for t in tensors:
         if t is not None and t.device.type != "cuda":
@@ -273,7 +285,8 @@ def _fwd_impl(q, k, v, key_mask, rope_cos, rope_sin, scale, key_tables=None):
     out = _kernel_ready(out)
     lse = torch.empty((B, Hq, Lq), device=q.device, dtype=torch.float32)
     lib = _lib.load()
-    ws = _workspace(lib.avattn_fwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D, 0), q.device)
+    ws = _split_workspace(lib.avattn_fwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D, 0),
+                          lambda: lib.avattn_fwd_workspace_size(B, Hkv, Lk, D), q.device)
     fwd, key_args = lib.avattn_fwd, ()
     if key_tables is not None:
         cos_k, sin_k, rksb = _check_tables(name, *key_tables, B, Lk, D)
@@ -345,7 +358,7 @@ def _fwd_f32_launch(name, q, k, v, lo, hi, wsb, key_mask, scale):
     lse = torch.empty((B, Hq, Lq), device=q.device, dtype=torch.float32)
     lib = _lib.load()
     need = lib.avattn_fwd_f32_split_workspace_size(B, Hq, Lq, Lk, D)
-    ws = _workspace(need, q.device) if need else None
+    ws = _split_workspace(need, lambda: 0, q.device) if need else None
     st = lib.avattn_fwd_f32_split(
         _ptr(q), _ptr(k), _ptr(v), _strides3(q), _strides3(k), _strides3(v),
         B, Hq, Hkv, Lq, Lk, D,
@@ -353,7 +366,7 @@ def _fwd_f32_launch(name, q, k, v, lo, hi, wsb, key_mask, scale):
         _ptr(lo), _ptr(hi), wsb,
         float(scale),
         _ptr(out), _strides3(out), _ptr(lse),
-        _ptr(ws), need,
+        _ptr(ws), 0 if ws is None else ws.numel(),
         _stream(q.device),
     )
     _lib.check(st, name)
@@ -413,21 +426,28 @@ def _alloc_bwd_f32_workspace(B, Hq, Hkv, Lq, Lk, device, D=None) -> torch.Tensor
     """The float32 backward's workspace: with the staged-dS budget (the one
     the bf16 backward uses) holding at least one (batch, kv head) pair's fp32
     dS, the staged size for as many pairs per pass as fit in equal passes
-    (halving while the allocator cannot provide it; all of them in one pass
-    with ``D`` given: also room for a split last dK/dV round), else the
-    statistics alone (dq recomputes S and dP)."""
+    (halving while the allocator cannot provide it), else the statistics alone
+    (dq recomputes S and dP).  With ``D`` given and all pairs in one pass also
+    room for a split last dK/dV round, if the budget and the allocator have
+    it."""
     lib = _lib.load()
-    pairs = 0
+    pairs = per = 0
     if B * Hkv > 0 and Lq > 0 and Lk > 0:
-        pairs = min(B * Hkv, _ds_budget(device) // f32_ds_bytes_per_pair(Hq // Hkv, Lq, Lk))
+        per = f32_ds_bytes_per_pair(Hq // Hkv, Lq, Lk)
+        pairs = min(B * Hkv, _ds_budget(device) // per)
     if pairs > 0:
         npass = -(-(B * Hkv) // pairs)
         pairs = -(-(B * Hkv) // npass)
+
+    def staged_size(p):
+        return lib.avattn_bwd_f32_staged_workspace_size(B, Hq, Hkv, Lq, Lk, int(p))
+
     while pairs > 0:
         try:
             if D is not None and pairs == B * Hkv:
-                return _workspace(lib.avattn_bwd_f32_split_workspace_size(B, Hq, Hkv, Lq, Lk, D), device)
-            return _workspace(lib.avattn_bwd_f32_staged_workspace_size(B, Hq, Hkv, Lq, Lk, int(pairs)), device)
+                split = lib.avattn_bwd_f32_split_workspace_size(B, Hq, Hkv, Lq, Lk, D)
+                return _one_pass_workspace(split, staged_size(pairs), int(pairs) * per, device)
+            return _workspace(staged_size(pairs), device)
         except torch.OutOfMemoryError:
             pairs = 0 if pairs == 1 else (pairs + 1) // 2
     return _workspace(lib.avattn_bwd_f32_workspace_size(B, Hq, Lq), device)
@@ -553,7 +573,8 @@ def _fwd_fp8_impl(q, k, v, key_mask, q_scale, k_scale, scale):
     out = _kernel_ready(torch.empty_like(q, memory_format=torch.preserve_format))
     lse = torch.empty((B, Hq, Lq), device=q.device, dtype=torch.float32)
     lib = _lib.load()
-    ws = _workspace(lib.avattn_fwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D, 1), q.device)
+    ws = _split_workspace(lib.avattn_fwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D, 1),
+                          lambda: lib.avattn_fwd_fp8_workspace_size(B, Hkv, Lk, D), q.device)
     st = lib.avattn_fwd_fp8(
         _ptr(q), _ptr(k), _ptr(v), _strides3(q), _strides3(k), _strides3(v),
         B, Hq, Hkv, Lq, Lk, D,
@@ -677,6 +698,15 @@ def _staged_pairs(B, Hq, Hkv, Lq, Lk, D, device, stage_ds=None, ds_units=0) -> i
     return -(-(B * Hkv) // npass)
 
 
+def _one_pass_workspace(split, staged, ds_bytes, device) -> torch.Tensor:
+    """The workspace of a backward with all its ``ds_bytes`` of dS in one pass:
+    ``split`` bytes, with room for the parts of a split dK/dV grid, if the dS
+    budget covers them and the allocator has them, else ``staged``."""
+    if ds_bytes + split - staged > _ds_budget(device):
+        return _workspace(staged, device)
+    return _split_workspace(split, lambda: staged, device)
+
+
 def bwd_workspace_plan(B, Hq, Hkv, Lq, Lk, D, device, stage_ds=None):
     """(bytes, staged) for one backward call: the workspace to allocate and
     whether dS is staged (``stage_ds`` None: when the staged dS of at least
@@ -694,23 +724,26 @@ def _alloc_bwd_workspace(B, Hq, Hkv, Lq, Lk, D, device, stage_ds=None, ds_units=
     """The workspace of :func:`bwd_workspace_plan`, allocated; if the caching
     allocator cannot provide it (memory held by activations, say), the
     staged pairs per pass halve until it can (more passes, the same
-    results), and with staging optional (``stage_ds`` not True) a last
-    attempt goes without staging (the recomputing dQ kernel).  ``ds_units``:
-    the compact layout of key windows (units per query head); ``windows``: key
-    windows in the dense layout.  All pairs in one pass without windows: also
-    room for a split dK/dV grid."""
+    results up to the order of fp32 sums in split key blocks), and with
+    staging optional (``stage_ds`` not True) a last attempt goes without
+    staging (the recomputing dQ kernel).  ``ds_units``: the compact layout of
+    key windows (units per query head); ``windows``: key windows in the dense
+    layout.  All pairs in one pass without windows: also room for a split
+    dK/dV grid, if the budget and the allocator have it."""
     lib = _lib.load()
     pairs = _staged_pairs(B, Hq, Hkv, Lq, Lk, D, device, stage_ds, ds_units)
 
     def staged_size(p):
         if ds_units:
             return lib.avattn_bwd_compact_workspace_size(B, Hq, Hkv, Lq, Lk, D, int(p), int(ds_units))
-        if p == B * Hkv and not windows:  # one pass: room for a split dK/dV grid too
-            return lib.avattn_bwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D)
         return lib.avattn_bwd_staged_workspace_size(B, Hq, Hkv, Lq, Lk, D, int(p))
 
     while pairs > 0:
         try:
+            if pairs == B * Hkv and not windows and not ds_units:
+                split = lib.avattn_bwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D)
+                ds_bytes = int(pairs) * ds_bytes_per_pair(Hq // Hkv, Lq, Lk)
+                return _one_pass_workspace(split, staged_size(pairs), ds_bytes, device)
             return _workspace(staged_size(pairs), device)
         except torch.OutOfMemoryError:
             if pairs == 1:
@@ -890,7 +923,8 @@ def _ring_fwd_step_impl(q, k, v, key_mask, cos_q, sin_q, cos_k, sin_k, scale, ou
     ck, sk, rksb = _ring_tables(name, cos_k, sin_k, B, Lk, D)
     flags = (_lib.RING_FIRST if first else 0) | (_lib.RING_LAST if last else 0)
     lib = _lib.load()
-    ws = _workspace(lib.avattn_fwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D, 0), q.device)
+    ws = _split_workspace(lib.avattn_fwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D, 0),
+                          lambda: lib.avattn_fwd_workspace_size(B, Hkv, Lk, D), q.device)
     st = lib.avattn_ring_fwd_step(
         _ptr(q), _ptr(k), _ptr(v), _strides3(q), _strides3(k), _strides3(v),
         B, Hq, Hkv, Lq, Lk, D,

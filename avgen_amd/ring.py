@@ -238,12 +238,13 @@ def _ring_backward_into(grad_out, query, key, value, out, lse, key_mask, cp, sca
     Hkv = key.shape[1]
     bounds = [shard_bounds(L, cp, r) for r in range(cp)]
     masks = [None if key_mask is None else key_mask[:, a:b] for a, b in bounds]
-    full = max(lib.avattn_bwd_split_workspace_size(B, Hq, Hkv, Lq, b - a, D) for a, b in bounds)
+    full = max(lib.avattn_bwd_staged_workspace_size(B, Hq, Hkv, Lq, b - a, D, B * Hkv) for a, b in bounds)
     if overlap and not (cp > 1 and full > 0):
         overlap = False
     if overlap:
         dev = query.device
-        ws = [ops._workspace(full, dev) for _ in range(2)]
+        split = max(lib.avattn_bwd_split_workspace_size(B, Hq, Hkv, Lq, b - a, D) for a, b in bounds)
+        ws = [ops._split_workspace(split, lambda: full, dev) for _ in range(2)]
         main = torch.cuda.current_stream(dev)
         side = torch.cuda.Stream(dev)
         done = [None, None]

@@ -7,7 +7,9 @@ functions and the host plan only; no launch).
 * passes are equal, the fewest that fit;
 * a workspace the allocator cannot provide is retried with half the pairs
   per pass down to one, then (staging optional) without staging, and raises
-  only where staging is required.
+  only where staging is required;
+* the room for a split grid is optional: it counts against the budget, and
+  where only it does not fit the call keeps its passes and runs unsplit.
 """
 
 from __future__ import annotations
@@ -111,3 +113,41 @@ def test_out_of_memory_falls_back_to_recompute_or_raises(device_props, monkeypat
     sizes.clear()
     ops._alloc_bwd_workspace(*shape, DEV, stage_ds=False)
     assert sizes == [base]
+
+
+F32 = (1, 20, 20, 4096, 4096, 128)  # 640 key blocks: a split last round
+
+
+def _bwd_sizes(lib, dtype):
+    if dtype == "f32":
+        return (F32, lib.avattn_bwd_f32_split_workspace_size(*F32),
+                lib.avattn_bwd_f32_staged_workspace_size(*F32[:5], 20), ops.f32_ds_bytes_per_pair(1, 4096, 4096),
+                lambda: ops._alloc_bwd_f32_workspace(*F32[:5], DEV, 128))
+    shape = (1, 20, 20, 10000, 128, 128)  # 20 key blocks: every one split
+    return (shape, lib.avattn_bwd_split_workspace_size(*shape), lib.avattn_bwd_staged_workspace_size(*shape, 20),
+            ops.ds_bytes_per_pair(1, 10000, 128), lambda: ops._alloc_bwd_workspace(*shape, DEV))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_room_for_a_split_is_optional(device_props, monkeypatch, dtype):
+    _, split, staged, per, alloc = _bwd_sizes(_lib.load(), dtype)
+    assert split > staged
+    sizes = _fake_alloc(monkeypatch, split)
+    assert alloc().numel() == split and sizes == [split]
+    sizes = _fake_alloc(monkeypatch, split - 1)  # only the parts do not fit: still one pass
+    assert alloc().numel() == staged and sizes == [split, staged]
+    sizes = _fake_alloc(monkeypatch, split)
+    ops.set_ds_budget(20 * per + split - staged, DEV)
+    assert alloc().numel() == split
+    ops.set_ds_budget(20 * per + split - staged - 1, DEV)  # the budget covers the dS alone
+    assert alloc().numel() == staged and sizes == [split, staged]
+
+
+def test_forward_workspace_falls_back_to_the_base_size(monkeypatch):
+    sizes = _fake_alloc(monkeypatch, 1000)
+    assert ops._split_workspace(1000, lambda: 600, DEV).numel() == 1000
+    assert ops._split_workspace(1001, lambda: 600, DEV).numel() == 600
+    assert sizes == [1000, 1001, 600]
+    for nbytes, base in ((1001, 1001), (2000, 1500)):
+        with pytest.raises(torch.OutOfMemoryError):
+            ops._split_workspace(nbytes, lambda: base, DEV)

@@ -62,3 +62,49 @@ def test_split_equals_unsplit(B, H, Lq, Lk, D, masked):
     if masked and B > 1:
         assert (o1[1] == 0).all()
     assert torch.equal(_call(lib, q, k, v, mask, split)[0].view(torch.int16), o1.view(torch.int16))
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp8", "ring", "f32"])
+def test_runs_unsplit_where_the_parts_do_not_fit(kind, monkeypatch):
+    """The parts' room is optional: an allocator that has the base workspace
+    only gives the unsplit call's bits."""
+    from avgen_amd import _lib, ops, ring
+    from avgen_amd.rope import RotaryTables
+
+    lib = _lib.load()
+    B, H, L, D = 1, 4, 2048, 128
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = (torch.randn(B, H, L, D, device="cuda", generator=g) for _ in range(3))
+    if kind != "f32":
+        q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+    s = 1.0 / math.sqrt(D)
+    ang = torch.randn(1, 1, L, D // 2, device="cuda", generator=g)
+    tables = RotaryTables(ang.cos(), ang.sin())
+
+    def call():
+        with torch.no_grad():
+            if kind == "fp8":
+                qs, ks = ops.fp8_absmax_scales(q), ops.fp8_absmax_scales(k)
+                return ops.flash_fwd_fp8(q, k, v, None, qs, ks, s)
+            if kind == "ring":
+                return ring.ring_attention(q, k, v, cp=1, tables_q=tables, tables_k=tables)
+            return ops.flash_fwd(q, k, v, None, None, None, s)
+
+    base = {"bf16": lib.avattn_fwd_workspace_size(B, H, L, D), "ring": lib.avattn_fwd_workspace_size(B, H, L, D),
+            "fp8": lib.avattn_fwd_fp8_workspace_size(B, H, L, D), "f32": 256}[kind]
+    real, sizes = ops._workspace, []
+
+    def small(nbytes, device):
+        sizes.append(nbytes)
+        if nbytes > base:
+            raise torch.OutOfMemoryError("no room for the parts")
+        return real(nbytes, device)
+
+    monkeypatch.setattr(ops, "_workspace", small)
+    got = call()
+    assert len(sizes) == 2 and sizes[0] > base >= sizes[1]
+    monkeypatch.setattr(ops, "_workspace", real)
+    name = "avattn_fwd_f32_split_workspace_size" if kind == "f32" else "avattn_fwd_split_workspace_size"
+    monkeypatch.setattr(lib, name, lambda *a: 0 if kind == "f32" else base)
+    for a, b in zip(got, call()):
+        assert torch.equal(a, b)
