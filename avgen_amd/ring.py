@@ -276,6 +276,12 @@ def _chunk_tables(tables, a, b):
     return None if tables is None else tables.slice(a, b)
 
 
+def _step_op(op, impl):
+    """A ring step: its implementation, or under a profiler the op, which its
+    trace names (in a call of Python's op layers each)."""
+    return op if torch.autograd._profiler_enabled() else impl
+
+
 def _ring_forward_fused(query, key, value, key_mask, cp, scale, tables_q, tables_k):
     """The emulated ring forward with RoPE and the merge fused into each
     chunk's launch (``ops.ring_fwd_step_``): q and k are unrotated, each
@@ -291,11 +297,11 @@ def _ring_forward_fused(query, key, value, key_mask, cp, scale, tables_q, tables
     acc = torch.empty(query.shape, dtype=torch.float32, device=query.device)
     lse = torch.empty((B, Hq, Lq), dtype=torch.float32, device=query.device)
     out = ops._kernel_ready(torch.empty_like(query, memory_format=torch.preserve_format))
+    step = _step_op(ops._ring_fwd_step_op, ops._ring_fwd_step_impl)
     for r, (a, b) in enumerate(bounds):
         tk = _chunk_tables(tables_k, a, b)
-        ops._ring_fwd_step_impl(query, key[:, :, a:b], value[:, :, a:b],
-                                None if key_mask is None else key_mask[:, a:b], tables_q.cos, tables_q.sin,
-                                tk.cos, tk.sin, scale, acc, lse, out, r == 0, r == cp - 1)
+        step(query, key[:, :, a:b], value[:, :, a:b], None if key_mask is None else key_mask[:, a:b], tables_q.cos,
+             tables_q.sin, tk.cos, tk.sin, scale, acc, lse, out, r == 0, r == cp - 1)
     return out, lse
 
 
@@ -317,12 +323,13 @@ def _ring_backward_fused(grad_out, query, key, value, out, lse, key_mask, cp, sc
     dq_acc = torch.zeros(query.shape, dtype=torch.float32, device=query.device)
     bounds = [shard_bounds(L, cp, r) for r in range(cp)]
     ws = _ring_workspace(B, Hq, Hkv, Lq, D, bounds, query.device)
+    step = _step_op(ops._ring_bwd_step_op, ops._ring_bwd_step_impl)
     for r, (a, b) in enumerate(bounds):
         tk = _chunk_tables(tables_k, a, b)
-        ops._ring_bwd_step_impl(grad_out, query, key[:, :, a:b], value[:, :, a:b], out, lse,
-                                None if key_mask is None else key_mask[:, a:b], tables_q.cos, tables_q.sin, tk.cos,
-                                tk.sin, scale, dq_acc, dk[:, :, a:b], dv[:, :, a:b], ws, r > 0)
-    ops._ring_dq_finish_impl(dq_acc, tables_q.cos, tables_q.sin, dq)
+        step(grad_out, query, key[:, :, a:b], value[:, :, a:b], out, lse,
+             None if key_mask is None else key_mask[:, a:b], tables_q.cos, tables_q.sin, tk.cos, tk.sin, scale, dq_acc,
+             dk[:, :, a:b], dv[:, :, a:b], ws, r > 0)
+    _step_op(ops._ring_dq_finish_op, ops._ring_dq_finish_impl)(dq_acc, tables_q.cos, tables_q.sin, dq)
     return dq, dk, dv
 
 

@@ -112,3 +112,15 @@ def test_batched_gradients_and_profiler_use_the_ops():
     with torch.autograd.profiler.profile() as prof:
         _run("flash_fwd", x)
     assert any("avgen_amd::flash_fwd" in e.name for e in prof.function_events)
+
+
+def test_a_profile_of_the_ring_names_its_steps():
+    x = _inputs(torch.bfloat16)
+    want = _run("ring_attention_rope", x)
+    with torch.autograd.profiler.profile() as prof:
+        got = _run("ring_attention_rope", x)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    names = [e.name for e in prof.function_events]
+    for name, count in (("ring_fwd_step", 2), ("ring_bwd_step", 2), ("ring_dq_finish", 1)):
+        assert names.count(f"avgen_amd::{name}") == count, name
