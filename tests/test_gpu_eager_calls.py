@@ -97,18 +97,30 @@ def test_saved_tensor_hooks_and_no_second_order(name):
         torch.autograd.grad(g.float().sum(), q)
 
 
-def test_batched_gradients_and_profiler_use_the_ops():
+@pytest.mark.parametrize("name", NAMES)
+def test_batched_gradients_use_the_ops(name, monkeypatch):
+    from avgen_amd import ops
+
     x = _inputs(torch.bfloat16)
     q = x["q"].clone().requires_grad_(True)
-    out = _calls()["rope_apply"]({**x, "q": q})
+    out = _calls()[name]({**x, "q": q})
     ref = [torch.autograd.grad(out, q, d, retain_graph=True)[0] for d in (x["do"], 2 * x["do"])]
-    got = None
-    try:
-        got = torch.autograd.grad(out, q, torch.stack([x["do"], 2 * x["do"]]), is_grads_batched=True)[0]
-    except RuntimeError:
-        pass  # no batching rule for the op: refused, never wrong
-    if got is not None:
-        assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
+    real, batched = ops._plain_eager, []
+
+    def spy(*tensors):
+        plain = real(*tensors)
+        if any(t is not None and "Batched" in str(torch._C._dispatch_keys(t)) for t in tensors):
+            batched.append(plain)
+        return plain
+
+    monkeypatch.setattr(ops, "_plain_eager", spy)
+    got = torch.autograd.grad(out, q, torch.stack([x["do"], 2 * x["do"]]), is_grads_batched=True)[0]
+    assert batched and not any(batched)
+    assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
+
+
+def test_profiled_calls_use_the_ops():
+    x = _inputs(torch.bfloat16)
     with torch.autograd.profiler.profile() as prof:
         _run("flash_fwd", x)
     assert any("avgen_amd::flash_fwd" in e.name for e in prof.function_events)

@@ -1,6 +1,7 @@
 """The forward with its last round split over ranges of keys against the
-unsplit one: the same result up to the rounding of the merge, and the row
-states (no attended key, NaN) merged exactly."""
+unsplit one, at every entry point that splits: the same result up to the
+rounding of the merge, and the row states (no attended key, NaN) merged
+exactly."""
 
 import math
 
@@ -62,6 +63,81 @@ def test_split_equals_unsplit(B, H, Lq, Lk, D, masked):
     if masked and B > 1:
         assert (o1[1] == 0).all()
     assert torch.equal(_call(lib, q, k, v, mask, split)[0].view(torch.int16), o1.view(torch.int16))
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("kind", ["rotated", "fp8", "ring first", "ring merge"])
+def test_entry_points_split_equals_unsplit(kind, D, masked):
+    """Grouped heads, q rotated, e4m3 scores (their own merge constants) and the
+    ring's fp32 accumulator, with parts that hold no attended key."""
+    from avgen_amd import _lib, ops
+
+    lib = _lib.load()
+    B, Hq, Hkv, Lq, Lk = 2, 4, 2, 700, 4097
+    g = torch.Generator(device="cuda").manual_seed(D)
+
+    def rnd(*shape):
+        return torch.randn(shape, device="cuda", generator=g)
+
+    q, k, v = rnd(B, Hq, Lq, D).bfloat16(), rnd(B, Hkv, Lk, D).bfloat16(), rnd(B, Hkv, Lk, D).bfloat16()
+    if kind == "fp8":
+        k[:, :, -1] *= 2  # the last part's reference is the largest
+    else:
+        q[0, 0, 5, 3] = float("nan")
+    mask = None
+    if masked:
+        mask = rnd(B, Lk) > -0.5
+        mask[:, : Lk // 2] = False
+        mask[1] = False
+        mask = mask.view(torch.uint8)
+    ang, angk = rnd(1, 1, Lq, D // 2), rnd(1, 1, Lk, D // 2)
+    tables = [t.contiguous() for t in (ang.cos(), ang.sin(), angk.cos(), angk.sin())]
+    qs, ks = (ops.fp8_absmax_scales(q), ops.fp8_absmax_scales(k)) if kind == "fp8" else (None, None)
+    acc0, lse0 = rnd(B, Hq, Lq, D), rnd(B, Hq, Lq)
+    lse0[:, :, ::3] = float("-inf")  # rows nothing was merged into yet
+    stream = torch.cuda.current_stream().cuda_stream
+    fp8 = int(kind == "fp8")
+    base = (lib.avattn_fwd_fp8_workspace_size if fp8 else lib.avattn_fwd_workspace_size)(B, Hkv, Lk, D)
+    split = lib.avattn_fwd_split_workspace_size(B, Hq, Hkv, Lq, Lk, D, fp8)
+    assert split > base
+
+    def call(nbytes):
+        out, lse = torch.empty_like(q), torch.empty((B, Hq, Lq), device="cuda")
+        acc, lacc = acc0.clone(), lse0.clone()
+        ws = torch.full((nbytes,), 255, dtype=torch.uint8, device="cuda")
+        head = (q.data_ptr(), k.data_ptr(), v.data_ptr(), ops._strides3(q), ops._strides3(k), ops._strides3(v), B, Hq,
+                Hkv, Lq, Lk, D, ops._ptr(mask), 0 if mask is None else Lk)
+        s = 1.0 / math.sqrt(D)
+        cq, sq, ck, sk = (t.data_ptr() for t in tables)
+        if kind == "rotated":
+            st = lib.avattn_fwd_rotary(*head, cq, sq, 0, ck, sk, 0, s, out.data_ptr(), ops._strides3(out),
+                                       lse.data_ptr(), ws.data_ptr(), nbytes, stream)
+        elif kind == "fp8":
+            st = lib.avattn_fwd_fp8(*head, qs.data_ptr(), ks.data_ptr(), s, out.data_ptr(), ops._strides3(out),
+                                    lse.data_ptr(), ws.data_ptr(), nbytes, stream)
+        else:
+            flags = _lib.RING_LAST | (_lib.RING_FIRST if kind == "ring first" else 0)
+            st = lib.avattn_ring_fwd_step(*head, cq, sq, 0, ck, sk, 0, s, acc.data_ptr(), lacc.data_ptr(),
+                                          out.data_ptr(), ops._strides3(out), flags, ws.data_ptr(), nbytes, stream)
+            lse = lacc
+        assert st == 0
+        return out, lse, acc
+
+    (o1, l1, a1), (o2, l2, a2) = call(split), call(base)
+    assert torch.equal(o1.isnan(), o2.isnan()) and torch.equal(l1.isnan(), l2.isnan())
+    assert torch.equal(l1 == float("-inf"), l2 == float("-inf"))
+    # as test_split_equals_unsplit; the ring adds the running output, exactly
+    d = (o1.float() - o2.float()).nan_to_num(0.0).abs()
+    assert (d <= 2.0**-7 * o2.float().nan_to_num(0.0).abs() + 2.0**-8).all()
+    if kind.startswith("ring"):
+        d = (a1 - a2).nan_to_num(0.0).abs()
+        assert (d <= 2.0**-7 * a2.nan_to_num(0.0).abs() + 2.0**-8).all()
+    f = torch.isfinite(l2)
+    assert (l1[f] - l2[f]).abs().max() <= 1e-5 * l2[f].abs().max()
+    if masked and kind != "ring merge":
+        rows = ~o1[1].isnan().any(-1)
+        assert (o1[1][rows] == 0).all() and (l1[1][rows] == float("-inf")).all()
 
 
 @pytest.mark.parametrize("kind", ["bf16", "fp8", "ring", "f32"])

@@ -94,3 +94,29 @@ def test_nan_query_row_without_keys_stays_nan():
     assert out[0, 0, 7].isnan().all() and lse[0, 0, 7].isnan()
     keep = torch.arange(Lq, device="cuda") != 7
     assert (out[0, 0, keep] == 0).all() and (lse[0, 0, keep] == -INF).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_masked_ends_in_several_passes(D):
+    """One (batch, kv head) pair of dS per pass: every pass leaves out its own
+    pair's tiles."""
+    from avgen_amd import _lib, ops
+
+    B, H, Hkv, Lq, L = 2, 4, 2, 150, 400
+    q, do = _rnd(B, H, Lq, D, seed=1), _rnd(B, H, Lq, D, seed=2)
+    k, v = _rnd(B, Hkv, L, D, seed=3), _rnd(B, Hkv, L, D, seed=4)
+    k[1, 1, 390, 7] = NAN  # this pair's last tile cannot be left out
+    key = torch.arange(L, device="cuda")
+    mask = torch.stack([(key >= 130) & (key < 200), key < 70])
+    s = 1.0 / math.sqrt(D)
+    out, lse = ops.flash_fwd(q, k, v, mask, None, None, s)
+    lib = _lib.load()
+    one, every = (ops._bwd_impl(do, q, k, v, out, lse, mask, s, stage_ds=True, workspace=torch.full(
+        (lib.avattn_bwd_staged_workspace_size(B, H, Hkv, Lq, L, D, n),), 255, dtype=torch.uint8, device="cuda"))
+        for n in (1, B * Hkv))
+    for label, a, b in zip(("dq", "dk", "dv"), one, every):
+        assert torch.equal(a.isnan(), b.isnan()), label
+        assert torch.equal(a.nan_to_num(0.0), b.nan_to_num(0.0)), label
+    assert torch.isfinite(one[0][0].float()).all() and one[0][1, 2:].isnan().any()
+    for g in one[1:]:
+        assert (g.transpose(1, 2)[~mask] == 0).all()
