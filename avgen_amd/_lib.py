@@ -335,7 +335,12 @@ def load() -> ctypes.CDLL:
             )
         lib = ctypes.CDLL(str(LIB_PATH))
         for name, (res, args) in SIGNATURES.items():
-            fn = getattr(lib, name)
+            fn = getattr(lib, name, None)
+            if fn is None:
+                raise RuntimeError(
+                    f"{LIB_PATH} has no {name}: it was built from older sources; rebuild it with "
+                    "`python -m avgen_amd.build`"
+                )
             fn.restype = res
             fn.argtypes = args
         _lib = lib

@@ -50,6 +50,14 @@ def test_every_declared_symbol_is_exported_and_bound(lib):
         assert hasattr(lib, name), name
 
 
+def test_a_library_without_an_entry_point_is_refused(lib, monkeypatch):
+    monkeypatch.setitem(_lib.SIGNATURES, "avattn_added_later", (ctypes.c_int, []))
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.raises(RuntimeError, match="no avattn_added_later: it was built from older sources"):
+        _lib.load()
+    assert _lib._lib is None
+
+
 def test_strerror_and_version(lib):
     assert lib.avattn_abi_version() == 14
     for code in range(0, 11):
