@@ -39,10 +39,12 @@ int check_dims(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lq, int32_t Lk, int32
   return AVATTN_OK;
 }
 
-// check_dims, plus the backward's own range: its dK/dV kernel stages the
-// padded q and dout rows of all query heads of one group through one 32-bit
-// buffer range each (group * Lqp * D bf16 below 2^32 bytes).  The forward
-// builds no range over q, so long grouped-query shapes stay valid there.
+// check_dims, plus the backward's own range.  The dK/dV kernel reads the row
+// statistics of all query heads of one group through one 32-bit buffer range
+// (group * Lqp floats; its Q and dO tiles have a range each).  The bound is
+// D / 2 times that, kept as the backward's limit on a group's padded rows
+// (group * Lqp * D bf16 below 2^32 bytes).  The forward builds no range over
+// q, so long grouped-query shapes are valid there.
 int check_bwd_dims(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lq, int32_t Lk, int32_t D) {
   const int st = check_dims(B, Hq, Hkv, Lq, Lk, D);
   if (st != AVATTN_OK || Hkv == 0 || Hq == 0) return st;
@@ -106,7 +108,9 @@ FwdWorkspace fwd_workspace(int32_t B, int32_t Hkv, int32_t Lk, int32_t D, bool f
 // Backward workspace: [lse2 | ndelta | q rows | dout rows |
 // k rows | v rows | k^T | key bias | key tile flags | dK/dV tail-split
 // partials (problems of more than 256 key blocks)], each region 256-byte
-// aligned.
+// aligned.  The size depends on sizes alone, so the row copies have their
+// regions also in calls that do not make them: q and dout read in place, k
+// and v with staged dS (whose khull and kskip are in the k rows' region).
 struct BwdWorkspace {
   size_t lse2, ndelta, qr, dor, kr, vr, kt, kbias, kfull, split, total;
 };

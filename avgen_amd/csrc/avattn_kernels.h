@@ -121,7 +121,9 @@ struct BwdArgs {
   float* lse2;    // lse * log2(e); +inf for rows with lse == -inf and padded rows
   // Padded copies (prep.hip) with H/Lp = Hq/Lqp (q, dout) or Hkv/Lkp
   // (k, v): row copies (*r) hold element (b, h, j, d) at ((b*H + h)*Lp + j)*D
-  // + d, head_dim-major copies (*t) at ((b*H + h)*D + d)*Lp + j.
+  // + d, head_dim-major copies (*t) at ((b*H + h)*D + d)*Lp + j.  qr and dor
+  // are written only where qt and dt point to them, kr and vr without staged
+  // dS.
   bf16* qr;
   bf16* dor;
   bf16* kr;
@@ -147,8 +149,7 @@ struct BwdArgs {
   // dq as an fp32 accumulator (dq_acc += this chunk's dq; dq is then null),
   // strides dqsb/dqsh/dqsl in floats.
   float* dq_acc;
-  // The query-side preparation (q/dout copies, lse2, ndelta) is already in
-  // the workspace: skip it.
+  // lse2, ndelta and a rotated q copy are already in the workspace: skip them.
   bool reuse_q;
   // Pass over the flattened (b, kv head) pairs kv0 .. kv0 + nkv - 1 (b*Hkv +
   // hk); the whole problem unless dS is staged in several passes.
@@ -297,7 +298,7 @@ inline int64_t transpose_padded_len(int64_t L) { return (L + 63) / 64 * 64; }
 // set everything but the K copy and kmax2).
 hipError_t launch_prep_fwd(const FwdArgs& a, int head_dim, hipStream_t stream);
 // The backward's (BwdArgs::kt, kbias, kfull, khull, the row copies it needs
-// and, unless a.reuse_q, lse2 and ndelta).
+// and, unless a.reuse_q, lse2 and ndelta; a.qt and a.dt must be set).
 hipError_t launch_prep_bwd(const BwdArgs& a, int head_dim, hipStream_t stream);
 
 // dq (bf16, strided) = transposed rotation of bf16(dq_acc) (fp32, strided);

@@ -81,7 +81,9 @@ typedef void* avattn_stream_t;
 /* Human-readable text for a status code (static storage, never NULL). */
 const char* avattn_strerror(int status);
 
-/* ABI version; bumped on any signature change. */
+/* ABI version; bumped on any change of a signature that exists.  Entry points
+ * are added under the same version: a program that looks them up at run time
+ * checks each; one linked against a library that lacks one does not load. */
 int avattn_abi_version(void);
 
 /*
@@ -150,7 +152,10 @@ int avattn_fwd_rotary(const void* q, const void* k, const void* v,
  * overlap on one GPU (concurrent streams, threads) share the array and race:
  * order them.  The first call on a device looks the array up
  * (hipGetSymbolAddress) and may return AVATTN_ERR_LAUNCH if that fails.
- * Every other argument and result is that of avattn_fwd, bit for bit.
+ * Every other argument and result is that of avattn_fwd with a workspace of
+ * avattn_fwd_workspace_size() bytes, bit for bit: the grid is never split, so
+ * the rows that avattn_fwd splits in a larger workspace
+ * (avattn_fwd_split_workspace_size()) differ from these in the last rounding.
  */
 #define AVATTN_FWD_NOALLOC_SCRATCH ((size_t)64 << 20)
 int avattn_fwd_noalloc(const void* q, const void* k, const void* v,
@@ -179,8 +184,11 @@ size_t avattn_fwd_workspace_size(int32_t batch, int32_t heads_kv, int32_t len_k,
  * grid over ranges of keys where that is faster: the base size plus the
  * parts' partial sums (0 for a problem the forward would refuse or that is
  * empty).  With a smaller workspace of at least the base size they run
- * unsplit; the split rows differ in the last rounding only.  Reproducible
- * bit for bit for a given workspace size either way.
+ * unsplit; the split rows differ in the last rounding only.  Which rows are
+ * split, and in how many parts, follows from every size here and the
+ * workspace size: the same (batch, head) slice may round differently in
+ * calls of other batch or head counts.  Reproducible bit for bit for given
+ * sizes either way.
  */
 size_t avattn_fwd_split_workspace_size(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t len_q, int32_t len_k,
                                        int32_t head_dim, int32_t fp8);
