@@ -1,7 +1,7 @@
 """The float32 kernels with a split last round (forward over keys, dK/dV over
 queries) against the unsplit ones: equal up to the order of fp32 sums, with
 NaN and infinite keys in the rows where the softmax has them; and dQ from
-staged dS at row counts around its workgroups' 128."""
+staged dS at row counts around its workgroups' 128 and 256."""
 
 import math
 
